@@ -193,8 +193,12 @@ int mi_matmul_lhs_rhs_bf16(const void* lhs, const void* rhs, void* out, int M, i
  * reference nkigym/src/nkigym/synthesis/simulate_nki.py:24-48).  Variant 0:
  * LDS-tiled FMAs, K summed in sequential order (64x64 blocks, block_k 16 or
  * 32); variant 1: the fp32 MFMA (v_mfma_f32_32x32x2_f32), K summed two at a
- * time (64x64 or 128x128 blocks, block_k 16).  Any M, N, K; 4-byte aligned
- * pointers; cfg == NULL selects mi_default_config. */
+ * time (64x64 or 128x128 blocks, block_k 16); variant 3: the fp32 MFMA with
+ * the K chunks of a block dealt to its waves, each summed two (16x16 blocks:
+ * four) at a time, then the waves' sums in wave order (16x16 blocks with
+ * block_k 32, 32- and 64-wide ones with 16, 2 stages, 4 to 16 waves;
+ * operands under 4 GiB).  There is no variant 2.  Any M, N, K; 4-byte
+ * aligned pointers; cfg == NULL selects mi_default_config. */
 int mi_matmul_lhsT_rhs_f32(const float* lhsT, const float* rhs, float* out, int M, int N, int K,
                            const mi_tile_cfg* cfg, void* stream);
 

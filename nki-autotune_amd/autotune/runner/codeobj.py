@@ -49,6 +49,7 @@ _TEMPLATES = {
     ("rmsnorm_matmul", 16): ("rmsnorm_mm_bf16_sq_pair_kernel", 5),
     ("matmul_lhsT_rhs_f32", 0): ("mm_f32_kernel", 3),
     ("matmul_lhsT_rhs_f32", 1): ("mm_f32_mfma_kernel", 2),
+    ("matmul_lhsT_rhs_f32", 3): ("mm_f32_kw_kernel", 4),
 }
 
 

@@ -109,12 +109,11 @@ bool splittable(int kernel_id, int variant) {
 namespace {
 
 using mi::capi::find;
+using mi::capi::kMaxOffset;
 using mi::capi::kMaxSplit;
 using mi::capi::kMaxWorkspace;
 using mi::capi::pick_default;
 using mi::capi::splittable;
-
-constexpr unsigned long long kMaxOffset = 0xFFFFFFFFull;        // 32-bit buffer offsets
 
 // The template rules of the variant `c` names (mi_legal.hpp: the same
 // predicates the kernel templates assert when they are instantiated).
@@ -153,6 +152,7 @@ mi::Legal template_legal(int kernel_id, const mi_tile_cfg& c) {
           return mi::bad(MI_E_TILE, "the fp32 MFMA kernel takes 64x64 or 128x128 blocks, block_k 16, 4 waves, 1 stage");
         return mi::ok();
       }
+      if (c.variant == 3) return mi::legal_f32_kw(bm, bn, bk, w, s);
       break;
     default:
       break;
@@ -228,6 +228,12 @@ int check(int kernel_id, const mi_tile_cfg* cfg, int M, int N, int K, const mi::
         return fail(MI_E_RANGE, "K=%d (%lld per part) exceeds the %d gamma entries variant %d stages in LDS", K,
                     need, e->gamma_kmax, c.variant);
     }
+  }
+  if (kernel_id == MI_KERNEL_MATMUL_LHST_RHS_F32 && c.variant == 3) {
+    const unsigned long long a_span = mi::capi::f32_kw_span(M, K, c.block_m);
+    const unsigned long long b_span = mi::capi::f32_kw_span(N, K, c.block_n);
+    if (a_span > kMaxOffset || b_span > kMaxOffset)
+      return fail(MI_E_RANGE, "operand spans exceed 32-bit buffer offsets (%llu, %llu bytes)", a_span, b_span);
   }
   if (out) *out = e;
   g_err[0] = '\0';

@@ -11,6 +11,15 @@ namespace capi {
 // Limits of a call: split-K parts, and bytes of device workspace.
 constexpr int kMaxSplit = 16;
 constexpr unsigned long long kMaxWorkspace = 1ull << 31;
+constexpr unsigned long long kMaxOffset = 0xFFFFFFFFull;  // 32-bit buffer offsets
+
+// Bytes that fp32 variant 3 addresses in an operand [K][cols] with blocks of
+// `block` columns: a K chunk's rows (at most 32) and a block's width from
+// each chunk's descriptor.
+inline unsigned long long f32_kw_span(int cols, int K, int block) {
+  const unsigned long long rows = (unsigned long long)(K > 32 ? K : 32);
+  return (rows * (unsigned long long)cols + (unsigned long long)block) * 4ull;
+}
 
 // Records the message of a failure for mi_last_error on this thread and
 // returns `code`.

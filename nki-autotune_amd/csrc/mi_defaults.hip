@@ -4,6 +4,8 @@
 // campaigns that timed every candidate block and split at about 200 more
 // shapes, and studies of 83 shapes and of seeded random ones.  Host code
 // only.
+#include <math.h>
+
 #include "mi_capi_internal.hpp"
 
 namespace mi {
@@ -424,6 +426,44 @@ mi_tile_cfg fused_default(int M, int N, int K) {
   return fastest_split_estimate(cands, n, M, N, K, mi_tile_cfg{128, 256, 64, 8, 2, 1, 8, 0});
 }
 
+// fp32: the MFMA kernel with K split over the waves (variant 3; variants 0,
+// in sequential K order, and 1 stay selectable), in the block and wave count
+// of the least estimated time (us).  The busiest CU runs `rounds` blocks.
+// Each costs its MFMAs (64 cycles per 4096 multiply-adds at 2.4 GHz and 0.94
+// of that rate; 0.42 for the 16x16 blocks, which wait for their loads more),
+// its operand bytes from L2 (63 GB/s per CU), and the latency of a load per
+// K chunk of a wave's chain (0.26 us, once: the rounds overlap); the three
+// overlap (their 3-norm), and the sum of the waves' blocks adds 6.1e-5 per
+// wave and output element.  Fitted to every candidate timed at 64 shapes
+// (M, N, K 64-4096, odd ones among them): the pick within 1.10 of the
+// fastest at all of them, 1.013 on average (the 64x64 block of variant 1:
+// 2.0 to 27 x the fastest).  A call whose operands pass 4 GiB, which variant
+// 3's 32-bit offsets do not reach, keeps variant 1.
+mi_tile_cfg f32_default(int M, int N, int K) {
+  static const mi_tile_cfg cands[] = {{64, 64, 16, 4, 2, 1, 8, 3},  {64, 32, 16, 4, 2, 1, 8, 3},
+                                      {32, 64, 16, 4, 2, 1, 8, 3},  {64, 32, 16, 8, 2, 1, 8, 3},
+                                      {32, 64, 16, 8, 2, 1, 8, 3},  {32, 32, 16, 8, 2, 1, 8, 3},
+                                      {32, 32, 16, 16, 2, 1, 8, 3}, {16, 16, 32, 4, 2, 1, 8, 3},
+                                      {16, 16, 32, 8, 2, 1, 8, 3},  {16, 16, 32, 16, 2, 1, 8, 3}};
+  if (f32_kw_span(M, K, 64) > kMaxOffset || f32_kw_span(N, K, 64) > kMaxOffset) return {64, 64, 16, 4, 1, 1, 0, 1};
+  mi_tile_cfg best = cands[0];
+  double best_t = 0.0;
+  for (const mi_tile_cfg& c : cands) {
+    const double rounds = (double)((tiles_of(M, N, c.block_m, c.block_n) + kCUs - 1) / kCUs);
+    const double chain = (double)(((K + c.block_k - 1) / c.block_k + c.waves - 1) / c.waves);  // chunks per wave
+    const double area = (double)c.block_m * c.block_n;
+    const double mfma = rounds * chain * (c.waves / 4) * c.block_k * area / 32.0 / 2400.0 / (c.block_m == 16 ? 0.42 : 0.94);
+    const double bytes = rounds * K * (double)(c.block_m + c.block_n) * 4.0 / 63e3;
+    const double wait = chain * 0.26;
+    const double t = cbrt(mfma * mfma * mfma + bytes * bytes * bytes + wait * wait * wait) + rounds * c.waves * area * 6.1e-5;
+    if (&c == cands || t < best_t) {
+      best = c;
+      best_t = t;
+    }
+  }
+  return best;
+}
+
 }  // namespace
 
 // The library default: the estimates and rules above, fitted to timed
@@ -432,8 +472,7 @@ int pick_default(int kernel_id, int M, int N, int K, mi_tile_cfg* cfg) {
   const bool lhs = kernel_id == MI_KERNEL_MATMUL_LHS_RHS_BF16;
   switch (kernel_id) {
     case MI_KERNEL_MATMUL_LHST_RHS_F32:
-      // The fp32 MFMA kernel; variant 0 (sequential K order) stays selectable.
-      *cfg = {64, 64, 16, 4, 1, 1, 0, 1};
+      *cfg = f32_default(M, N, K);
       break;
     case MI_KERNEL_MATMUL_LHST_RHS_BF16:
     case MI_KERNEL_MATMUL_LHS_RHS_BF16:

@@ -156,6 +156,25 @@ MI_HD constexpr Legal legal_mm_kw(int bm, int bn, int bk, int waves, int stages)
   return ok();
 }
 
+// ---- fp32 lhsT.rhs with K split over the waves (fp32 variant 3): every
+// wave holds the whole block's accumulators and two K chunks of block_k rows
+// of both operands in registers, and an LDS slot for its block (rows padded
+// by 4) in the sum.
+MI_HD constexpr int lds_f32_kw(int bm, int bn, int waves) { return waves * bm * (bn + 4) * 4; }
+MI_HD constexpr Legal legal_f32_kw(int bm, int bn, int bk, int waves, int stages) {
+  // 16x16 blocks of 16x16x4 MFMAs; 32- and 64-wide ones of 32x32x2 MFMAs.
+  const bool small = bm == 16 && bn == 16 && bk == 32;
+  const bool large = (bm == 32 || bm == 64) && (bn == 32 || bn == 64) && bk == 16;
+  if ((!small && !large) || stages != 2)
+    return bad(MI_E_TILE, "the fp32 kernel with K split over the waves takes 16x16 blocks with block_k 32, or 32- and "
+                          "64-wide blocks with block_k 16, 2 stages");
+  if (waves != 4 && waves != 8 && waves != 16) return bad(MI_E_WAVE_TILE, "4, 8 or 16 waves split K");
+  if ((bm * bn / 64 + bk * (bm + bn) / 32 + bk + 30) * (waves / 4) > 512)
+    return bad(MI_E_WAVE_TILE, "accumulators and operand chunks exceed a wave's share of the 512 registers");
+  if (lds_f32_kw(bm, bn, waves) > kLdsBytesMax) return bad(MI_E_LDS, "LDS over 160 KiB");
+  return ok();
+}
+
 // ---- main pass of the two-pass fused kernel (rmsnorm_matmul variant 13):
 // the pipelined lhsT.rhs core plus the block's BM row scales in LDS.
 MI_HD constexpr int lds_rms2(int bm, int bn, int bk, int waves, int stages) {
