@@ -3,7 +3,9 @@
 Every ``*.hip`` translation unit under ``csrc/`` is compiled ahead of time
 with ``hipcc --offload-arch=gfx950`` (in parallel, one process per unit) and
 linked into ``kernel_library/libmi_kernels.so``, which the ctypes loader in
-``kernel_library/_lib.py`` opens.  The tile-config search space lives in the
+``kernel_library/_lib.py`` opens.  ``csrc/host/`` holds the native half of
+the torch call (a CPython extension over torch's C++ headers, host code
+only), built into ``kernel_library/_torch_call.so``.  The tile-config search space lives in the
 instance tables of those units, so building the library is the "compile"
 step of every autotune candidate at once.  The units under ``csrc/probe/``
 (measurement probes for bench.py, outside the kernel_library ABI) are linked
@@ -19,6 +21,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -27,6 +30,7 @@ CSRC = PKG_DIR / "csrc"
 BUILD = PKG_DIR / "_build"
 LIB = PKG_DIR / "kernel_library" / "libmi_kernels.so"
 PROBE_LIB = PKG_DIR / "kernel_library" / "libmi_probe.so"
+TORCH_CALL = PKG_DIR / "kernel_library" / "_torch_call.so"
 INCLUDE = PKG_DIR.parent / "include"
 
 ARCH = "gfx950"
@@ -83,8 +87,30 @@ def _link(objs: list[Path], lib: Path) -> None:
     os.replace(tmp, lib)
 
 
+def _build_torch_call(force: bool) -> None:
+    """csrc/host/mi_torch_call.cpp -> kernel_library/_torch_call.so (g++ against the installed torch)."""
+    src = CSRC / "host" / "mi_torch_call.cpp"
+    deps = [src, *INCLUDE.glob("*.h")]
+    if not force and TORCH_CALL.exists() and TORCH_CALL.stat().st_mtime >= max(p.stat().st_mtime for p in deps):
+        return
+    import torch
+    from torch.utils import cpp_extension
+
+    # torch's HIP headers ask the host compiler which platform they are for.
+    flags = ["-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+    paths = [*cpp_extension.include_paths("cuda"), sysconfig.get_paths()["include"]]
+    tmp = TORCH_CALL.with_suffix(".so.tmp")
+    cmd = ["g++", *flags, *(f"-I{p}" for p in paths), str(src), "-o", str(tmp),
+           f"-L{Path(torch.__file__).parent / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed for {src.name}:\n{proc.stdout}{proc.stderr}")
+    os.replace(tmp, TORCH_CALL)
+
+
 def build(jobs: int | None = None, force: bool = False, verbose: bool = False) -> Path:
-    """Compile every csrc/*.hip unit and link libmi_kernels.so (and csrc/probe/ into libmi_probe.so)."""
+    """Compile every csrc/*.hip unit and link libmi_kernels.so (csrc/probe/: libmi_probe.so; csrc/host/: _torch_call.so)."""
     BUILD.mkdir(parents=True, exist_ok=True)
     srcs = _sources()
     if not srcs:
@@ -92,7 +118,9 @@ def build(jobs: int | None = None, force: bool = False, verbose: bool = False) -
     probes = sorted((CSRC / "probe").glob("*.hip"))
     jobs = jobs or max(1, min(len(srcs) + len(probes), (os.cpu_count() or 2)))
     with ThreadPoolExecutor(max_workers=jobs) as pool:
+        torch_call = pool.submit(_build_torch_call, force)
         results = list(pool.map(lambda s: _compile(s, force), srcs + probes))
+    torch_call.result()
     if verbose:
         for obj, log in results:
             if log.strip():

@@ -11,8 +11,10 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <atomic>
 #include <map>
 #include <mutex>
+#include <unordered_map>
 #include <utility>
 #include <vector>
 
@@ -59,9 +61,25 @@ const std::vector<mi::MiEntry>& registry() {
   return all;
 }
 
-bool same_instance(const mi_tile_cfg& a, const mi_tile_cfg& b) {
-  return a.block_m == b.block_m && a.block_n == b.block_n && a.block_k == b.block_k && a.waves == b.waves &&
-         a.lds_stages == b.lds_stages && a.variant == b.variant;
+// The instance fields of a config in one word; 0 when a field is outside
+// what any instance has (every call looks its instance up).
+uint64_t instance_key(int kernel_id, const mi_tile_cfg& c) {
+  const int f[] = {c.block_m, c.block_n, c.block_k, c.waves, c.lds_stages, c.variant};
+  uint64_t key = (uint64_t)kernel_id + 1;
+  for (const int v : f) {
+    if (v < 0 || v >= 1024) return 0;
+    key = key << 10 | (uint64_t)v;
+  }
+  return key;
+}
+
+const std::unordered_map<uint64_t, const mi::MiEntry*>& instance_index() {
+  static const auto* index = [] {
+    auto* m = new std::unordered_map<uint64_t, const mi::MiEntry*>;
+    for (const mi::MiEntry& e : registry()) m->emplace(instance_key(e.kernel_id, e.cfg), &e);
+    return m;
+  }();
+  return *index;
 }
 
 }  // namespace
@@ -70,30 +88,30 @@ namespace mi {
 namespace capi {
 
 const MiEntry* find(int kernel_id, const mi_tile_cfg& cfg) {
-  for (const MiEntry& e : registry())
-    if (e.kernel_id == kernel_id && same_instance(e.cfg, cfg)) return &e;
-  return nullptr;
+  const uint64_t key = instance_key(kernel_id, cfg);
+  const auto it = key ? instance_index().find(key) : instance_index().end();
+  return it == instance_index().end() ? nullptr : it->second;
 }
 
 int device_cus() {
-  static std::mutex mu;
-  static std::map<int, int> cus;
+  constexpr int kDevices = 64;
+  static std::atomic<int> cus[kDevices];  // 0: not asked yet
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) {
     (void)hipGetLastError();  // no device (a CPU-only host): leave no error behind for a later launch check
     return kDefaultCus;
   }
-  std::lock_guard<std::mutex> lock(mu);
-  auto it = cus.find(dev);
-  if (it == cus.end()) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) {
-      (void)hipGetLastError();
-      n = kDefaultCus;
-    }
-    it = cus.emplace(dev, n).first;
+  if (dev >= 0 && dev < kDevices) {
+    const int known = cus[dev].load(std::memory_order_relaxed);
+    if (known > 0) return known;
   }
-  return it->second;
+  int n = 0;
+  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) {
+    (void)hipGetLastError();
+    n = kDefaultCus;
+  }
+  if (dev >= 0 && dev < kDevices) cus[dev].store(n, std::memory_order_relaxed);
+  return n;
 }
 
 bool splittable(int kernel_id, int variant) {

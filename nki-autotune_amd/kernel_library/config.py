@@ -16,7 +16,9 @@ import json
 from dataclasses import asdict, dataclass, replace
 from pathlib import Path
 
-from kernel_library import _lib
+import torch  # noqa: F401  (loads the libraries that _torch_call links)
+
+from kernel_library import _lib, _torch_call
 
 KERNEL_IDS = {
     "matmul_lhsT_rhs": _lib.MI_KERNEL_MATMUL_LHST_RHS_BF16,
@@ -247,6 +249,7 @@ def tuned_table(reload: bool = False) -> dict:
     global _TABLE_CACHE
     if _TABLE_CACHE is None or reload:
         _DEFAULT_CACHE.clear()
+        _torch_call.forget()
         data = {}
         if TUNED_TABLE.exists():
             data = json.loads(TUNED_TABLE.read_text()).get("configs", {})

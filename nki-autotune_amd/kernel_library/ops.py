@@ -18,18 +18,37 @@ Drop-in for the reference kernel_library call signatures:
 Shape mismatches raise ``ValueError`` (the reference asserts its fixed
 shapes, :103-104).  Every call runs a HIP kernel from libmi_kernels.so on the
 current torch stream; there is no fallback path.
+
+A call without a config first goes to ``_torch_call.call``
+(csrc/host/mi_torch_call.cpp), which does the steps of the Python body below
+in native code for plain contiguous tensors at a shape whose config it was
+given, and returns None for everything else.
 """
 
 from __future__ import annotations
 
 import ctypes
+import os
 
 import torch
 
-from kernel_library import _lib
+from kernel_library import _lib, _torch_call
 from kernel_library.config import TileConfig, default_config
 
 EPS = 1e-6
+
+# Kinds of _torch_call (csrc/host/mi_torch_call.cpp); lhsT.rhs in fp32 is kind 1 of its table.
+_LHST, _LHST_F32, _RMS, _LHS, _RMS_NO_GAMMA = range(5)
+
+
+def _remember(kind: int, M: int, N: int, K: int, cfg: TileConfig) -> None:
+    """Hand the native call the config that this shape has just run with, and the library that ran it."""
+    L = _lib.lib()
+    fns = (L.mi_matmul_lhsT_rhs_bf16, L.mi_matmul_lhsT_rhs_f32, L.mi_rmsnorm_matmul_bf16, L.mi_matmul_lhs_rhs_bf16)
+    _torch_call.bind(os.environ.get("MI_KERNELS_LIB", ""), *(ctypes.cast(f, ctypes.c_void_p).value for f in fns),
+                     _lib.check_rc)
+    _torch_call.remember(kind, M, N, K, cfg.block_m, cfg.block_n, cfg.block_k, cfg.waves, cfg.lds_stages, cfg.split_k,
+                         cfg.group_m, cfg.variant)
 
 
 def _stream_handle(device: torch.device) -> int:
@@ -75,6 +94,10 @@ def matmul_lhsT_rhs(
     out: torch.Tensor | None = None,
 ) -> torch.Tensor:
     """``out[M,N] = lhs_T[K,M].T @ rhs[K,N]`` on the GPU (bf16 or fp32)."""
+    if cfg is None:
+        done = _torch_call.call(_LHST, lhs_T, rhs, None, 0.0, out)
+        if done is not None:
+            return done
     _check_operand("lhs_T", lhs_T, (torch.bfloat16, torch.float32))
     _check_operand("rhs", rhs, (torch.bfloat16, torch.float32))
     if lhs_T.dtype != rhs.dtype:
@@ -92,14 +115,16 @@ def matmul_lhsT_rhs(
         _no_overlap(out, lhs_T=lhs_T, rhs=rhs)
     fp32 = lhs_T.dtype == torch.float32
     name = "matmul_lhsT_rhs_f32" if fp32 else "matmul_lhsT_rhs"
-    cfg = cfg if cfg is not None else default_config(name, M, N, K)
-    c = cfg.to_c()
+    use = cfg if cfg is not None else default_config(name, M, N, K)
+    c = use.to_c()
     L = _lib.lib()
     fn = L.mi_matmul_lhsT_rhs_f32 if fp32 else L.mi_matmul_lhsT_rhs_bf16
     with torch.cuda.device(lhs_T.device):
         rc = fn(lhs_T.data_ptr(), rhs.data_ptr(), out.data_ptr(), M, N, K, ctypes.byref(c),
                 _stream_handle(lhs_T.device))
     _lib.check_rc(rc, name)
+    if cfg is None:
+        _remember(_LHST_F32 if fp32 else _LHST, M, N, K, use)
     return out
 
 
@@ -110,6 +135,10 @@ def matmul_lhs_rhs(
     out: torch.Tensor | None = None,
 ) -> torch.Tensor:
     """``out[M,N] = lhs[M,K] @ rhs[K,N]`` on the GPU (bf16, lhs K-contiguous)."""
+    if cfg is None:
+        done = _torch_call.call(_LHS, lhs, rhs, None, 0.0, out)
+        if done is not None:
+            return done
     _check_operand("lhs", lhs, (torch.bfloat16,))
     _check_operand("rhs", rhs, (torch.bfloat16,))
     _same_device("lhs", lhs, rhs=rhs, out=out)
@@ -123,12 +152,14 @@ def matmul_lhs_rhs(
         raise ValueError(f"out must be a contiguous bf16 [{M},{N}] tensor")
     else:
         _no_overlap(out, lhs=lhs, rhs=rhs)
-    cfg = cfg if cfg is not None else default_config("matmul_lhs_rhs", M, N, K)
-    c = cfg.to_c()
+    use = cfg if cfg is not None else default_config("matmul_lhs_rhs", M, N, K)
+    c = use.to_c()
     with torch.cuda.device(lhs.device):
         rc = _lib.lib().mi_matmul_lhs_rhs_bf16(lhs.data_ptr(), rhs.data_ptr(), out.data_ptr(), M, N, K,
                                                ctypes.byref(c), _stream_handle(lhs.device))
     _lib.check_rc(rc, "matmul_lhs_rhs")
+    if cfg is None:
+        _remember(_LHS, M, N, K, use)
     return out
 
 
@@ -141,6 +172,10 @@ def rmsnorm_matmul(
     out: torch.Tensor | None = None,
 ) -> torch.Tensor:
     """``out[M,N] = (lhs[M,K] / sqrt(mean_k lhs^2 + eps) * gamma[K]) @ rhs[K,N]`` (bf16)."""
+    if cfg is None:
+        done = _torch_call.call(_RMS, lhs, rhs, gamma, eps, out)
+        if done is not None:
+            return done
     _check_operand("lhs", lhs, (torch.bfloat16,))
     _check_operand("rhs", rhs, (torch.bfloat16,))
     _same_device("lhs", lhs, rhs=rhs, gamma=gamma, out=out)
@@ -158,16 +193,18 @@ def rmsnorm_matmul(
         raise ValueError(f"out must be a contiguous bf16 [{M},{N}] tensor")
     else:
         _no_overlap(out, lhs=lhs, rhs=rhs, gamma=gamma)
-    if cfg is None:
-        # Without gamma (the reference's contract) the no-gamma default: its
-        # own tuned winner for the shape first.
-        cfg = default_config("rmsnorm_matmul_online" if gamma is None else "rmsnorm_matmul", M, N, K)
-    c = cfg.to_c()
+    # Without gamma (the reference's contract) the no-gamma default: its own
+    # tuned winner for the shape first.
+    use = cfg if cfg is not None else default_config("rmsnorm_matmul_online" if gamma is None else "rmsnorm_matmul",
+                                                     M, N, K)
+    c = use.to_c()
     gptr = gamma.data_ptr() if gamma is not None else None
     with torch.cuda.device(lhs.device):
         rc = _lib.lib().mi_rmsnorm_matmul_bf16(lhs.data_ptr(), gptr, rhs.data_ptr(), out.data_ptr(), M, N, K,
                                                float(eps), ctypes.byref(c), _stream_handle(lhs.device))
     _lib.check_rc(rc, "rmsnorm_matmul")
+    if cfg is None:
+        _remember(_RMS if gamma is not None else _RMS_NO_GAMMA, M, N, K, use)
     return out
 
 
