@@ -656,26 +656,54 @@ __device__ __forceinline__ void kw_reduce_store(const f32x16_t (&acc)[TM][TN], c
   }
 }
 
+// v[0] + v[stride] + ... + v[(parts - 1) * stride], added in that order.
+// PARTS > 0 is the count, known at compile time; PARTS == 0 takes `parts`,
+// eight at a time.  Every load of a group is issued before the first sum:
+// the parts were written by other CUs, so each is a trip past the L2, and a
+// loop that adds a part before it loads the next makes that trip once per
+// part (16 parts: 9.8 us for 48 x 232 outputs, 3.0 with the loads together).
+template <int PARTS, class T>
+__device__ __forceinline__ T sum_in_order(const T* __restrict__ v, size_t stride, int parts) {
+  if constexpr (PARTS > 0) {
+    T x[PARTS];
+#pragma unroll
+    for (int p = 0; p < PARTS; ++p) x[p] = *(const T*)((const char*)v + (size_t)p * stride * sizeof(float));
+    T s = x[0];
+#pragma unroll
+    for (int p = 1; p < PARTS; ++p) s += x[p];
+    return s;
+  } else {
+    constexpr int G = 8;
+    T s{};
+    for (int p0 = 0; p0 < parts; p0 += G) {
+      T x[G];
+#pragma unroll
+      for (int q = 0; q < G; ++q) {
+        const int p = p0 + q < parts ? p0 + q : parts - 1;
+        x[q] = *(const T*)((const char*)v + (size_t)p * stride * sizeof(float));
+      }
+#pragma unroll
+      for (int q = 0; q < G; ++q)
+        if (p0 + q < parts) s = p0 + q == 0 ? x[q] : s + x[q];
+    }
+    return s;
+  }
+}
+
 // out[i] = bf16(sum over p = 0 .. parts-1 of ws[p][i]), summed in part order
-// (so the result does not depend on the order the parts ran in); 8
+// (so the result does not depend on the order the parts ran in); 4
 // elements per thread (n = M*N, a multiple of 8).  A template so that every
 // translation unit may instantiate it.
-template <int UNUSED = 0>
+template <int PARTS>
 __global__ __launch_bounds__(256) void splitk_sum_kernel(const float* __restrict__ ws, uint16_t* __restrict__ out,
                                                          size_t n, int parts) {
-  const size_t stride = (size_t)gridDim.x * 256 * 8;
-  for (size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 8; i < n; i += stride) {
-    f32x4_t lo = *(const f32x4_t*)(ws + i), hi = *(const f32x4_t*)(ws + i + 4);
-    for (int p = 1; p < parts; ++p) {
-      lo += *(const f32x4_t*)(ws + (size_t)p * n + i);
-      hi += *(const f32x4_t*)(ws + (size_t)p * n + i + 4);
-    }
-    u32x4_t o;
-    o.x = pack_bf16x2(lo[0], lo[1]);
-    o.y = pack_bf16x2(lo[2], lo[3]);
-    o.z = pack_bf16x2(hi[0], hi[1]);
-    o.w = pack_bf16x2(hi[2], hi[3]);
-    *(u32x4_t*)(out + i) = o;
+  const size_t stride = (size_t)gridDim.x * blockDim.x * 4;
+  for (size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 4; i < n; i += stride) {
+    const f32x4_t s = sum_in_order<PARTS>((const f32x4_t*)(ws + i), n, parts);
+    u32x2_t o;
+    o.x = pack_bf16x2(s[0], s[1]);
+    o.y = pack_bf16x2(s[2], s[3]);
+    *(u32x2_t*)(out + i) = o;
   }
 }
 

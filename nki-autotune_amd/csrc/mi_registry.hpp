@@ -93,20 +93,44 @@ hipError_t launch_mm_bf16(const MiArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+// The second pass of split-K takes 4 outputs per thread: blocks of 256
+// threads where that fills the CUs, of 64 where the output is smaller (so
+// that its loads, which are latency, come from four times as many CUs).
+struct SumGrid {
+  dim3 grid, block;
+};
+inline SumGrid splitk_sum_grid(size_t n) {
+  const size_t threads = n / 4;
+  const unsigned block = threads >= 256 * 256 ? 256 : 64;
+  const size_t blocks = (threads + block - 1) / block;
+  return SumGrid{dim3((unsigned)(blocks < 8192 ? blocks : 8192)), dim3(block)};
+}
+
 // Split-K second pass: out = bf16(sum over the parts of ws), in part order.
 inline void launch_splitk_sum(const float* ws, uint16_t* out, size_t n, int parts, hipStream_t s) {
-  const size_t blocks = (n / 8 + 255) / 256;
-  hipLaunchKernelGGL(splitk_sum_kernel<0>, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s, ws, out,
-                     n, parts);
+  const SumGrid g = splitk_sum_grid(n);
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, g.grid, g.block, 0, s, ws, out, n, parts); };
+  if (parts == 2) go(splitk_sum_kernel<2>);
+  else if (parts == 4) go(splitk_sum_kernel<4>);
+  else if (parts == 8) go(splitk_sum_kernel<8>);
+  else if (parts == 16) go(splitk_sum_kernel<16>);
+  else go(splitk_sum_kernel<0>);
 }
 
 // Split-K second pass of the fused kernels: products and sums of squares in
 // part order, then 1/rms and the bf16 rounding.
 inline void launch_splitk_rms_sum(const float* prod, int parts, const float* ssq, int ssq_parts, const MiArgs& a,
                                   hipStream_t s) {
-  const size_t blocks = ((size_t)a.M * (size_t)a.N / 8 + 255) / 256;
-  hipLaunchKernelGGL(splitk_rms_sum_kernel<0>, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s,
-                     prod, (uint16_t*)a.out, a.M, a.N, parts, ssq, ssq_parts, a.inv_k, a.eps);
+  const SumGrid g = splitk_sum_grid((size_t)a.M * (size_t)a.N);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, g.grid, g.block, 0, s, prod, (uint16_t*)a.out, a.M, a.N, parts, ssq, ssq_parts, a.inv_k,
+                       a.eps);
+  };
+  if (parts == 2) go(splitk_rms_sum_kernel<2>);
+  else if (parts == 4) go(splitk_rms_sum_kernel<4>);
+  else if (parts == 8) go(splitk_rms_sum_kernel<8>);
+  else if (parts == 16) go(splitk_rms_sum_kernel<16>);
+  else go(splitk_rms_sum_kernel<0>);
 }
 
 template <int BM, int BN, int BK, int W, int S, bool NTB = false>

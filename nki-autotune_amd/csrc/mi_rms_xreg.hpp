@@ -393,32 +393,26 @@ __global__ __launch_bounds__(WAVES * 64) void rmsnorm_mm_bf16_xreg_kernel(
   store_tile<TM, TN, WAVES>(acc, scale, smem, wave, lane, out, M, N, m0 + wm0, n0 + wn0);
 }
 
-// Split-K second pass of the fused kernel: for 8 consecutive elements of
+// Split-K second pass of the fused kernel: for 4 consecutive elements of
 // row m, out = bf16(rsqrt(sum_q ssq[q][m] * inv_k + eps) * sum_p ws[p][...]),
 // both sums in part order (ws = [parts][M][N] products, ssq = [ssq_parts][M]
-// partial sums of squares; N % 8 == 0, so 8 elements never straddle rows).
-template <int UNUSED = 0>
+// partial sums of squares; N % 8 == 0, so 4 elements never straddle rows,
+// and M * N < 2^32, as [parts][M][N] fits the 2 GiB a workspace may have).
+template <int PARTS>
 __global__ __launch_bounds__(256) void splitk_rms_sum_kernel(const float* __restrict__ ws, uint16_t* __restrict__ out,
                                                              int M, int N, int parts, const float* __restrict__ ssq,
                                                              int ssq_parts, float inv_k, float eps) {
   const size_t n = (size_t)M * (size_t)N;
-  const size_t stride = (size_t)gridDim.x * 256 * 8;
-  for (size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 8; i < n; i += stride) {
-    const size_t m = i / (size_t)N;
-    float r = ssq[m];
-    for (int q = 1; q < ssq_parts; ++q) r += ssq[(size_t)q * M + m];
-    f32x4_t lo = *(const f32x4_t*)(ws + i), hi = *(const f32x4_t*)(ws + i + 4);
-    for (int p = 1; p < parts; ++p) {
-      lo += *(const f32x4_t*)(ws + (size_t)p * n + i);
-      hi += *(const f32x4_t*)(ws + (size_t)p * n + i + 4);
-    }
+  const size_t stride = (size_t)gridDim.x * blockDim.x * 4;
+  for (size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 4; i < n; i += stride) {
+    const uint32_t m = (uint32_t)i / (uint32_t)N;
+    const f32x4_t s = sum_in_order<PARTS>((const f32x4_t*)(ws + i), n, parts);
+    const float r = sum_in_order<0>(ssq + m, (size_t)M, ssq_parts);
     const float sc = 1.0f / __builtin_sqrtf(r * inv_k + eps);
-    u32x4_t o;
-    o.x = pack_bf16x2(lo[0] * sc, lo[1] * sc);
-    o.y = pack_bf16x2(lo[2] * sc, lo[3] * sc);
-    o.z = pack_bf16x2(hi[0] * sc, hi[1] * sc);
-    o.w = pack_bf16x2(hi[2] * sc, hi[3] * sc);
-    *(u32x4_t*)(out + i) = o;
+    u32x2_t o;
+    o.x = pack_bf16x2(s[0] * sc, s[1] * sc);
+    o.y = pack_bf16x2(s[2] * sc, s[3] * sc);
+    *(u32x2_t*)(out + i) = o;
   }
 }
 
