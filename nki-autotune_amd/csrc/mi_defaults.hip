@@ -426,6 +426,184 @@ mi_tile_cfg fused_default(int M, int N, int K) {
   return fastest_split_estimate(cands, n, M, N, K, mi_tile_cfg{128, 256, 64, 8, 2, 1, 8, 0});
 }
 
+// Fitted times.  A candidate's time (us) at a shape is
+//   start + (tile + step * L * (1 + crowd * f)) * (1 + (n - 1) * more)
+//   + read_mb * (the inputs' MB)
+//   [+ split + split_mb * p * M * N / 1e6]      K split in p parts
+//   [+ pack + pack_mb * M * K / 1e6]            the two-pass fused kernels
+// with L the K tiles of a part, n the workgroups of the busiest CU, and f
+// the share of CUs that have one (at most 1): one tile's fixed cost, its cost
+// per K tile (more when every CU loads at once), and the further tiles of a
+// CU, which overlap the first one's loads.  The coefficients are fitted to
+// every candidate block in 1-8, 12 and 16 parts, timed at 480 fused, 320
+// no-gamma, 380 lhsT.rhs and 380 lhs.rhs shapes with M > 128 (sizes spread
+// over their logarithm, N up to 28672, K up to 16384), three sets of inputs
+// in turn.  Fitted without half of the second campaigns' shapes, the least
+// fitted time is within 1.012, 1.023, 1.022 and 1.021 of the fastest on
+// average at those.
+struct Timed {
+  mi_tile_cfg c;
+  double start, tile, step, more, crowd, read_mb, split, split_mb, pack, pack_mb;
+};
+
+const Timed kFusedTimed[] = {
+    {{128, 512, 32, 8, 3, 1, 8, 4}, 1.39, 5.75, 0.444, 1.04, 0.744, 0.0336, 2.4, 1.06, 0, 0},
+    {{128, 128, 64, 4, 2, 1, 8, 4}, 1.78, 3.33, 0.525, 0.933, 0.26, 0.0192, 2.86, 1.32, 0, 0},
+    {{256, 128, 32, 8, 3, 1, 8, 5}, 1.83, 3.93, 0.375, 1.05, 0.468, 0.0166, 3.92, 1.04, 0, 0},
+    {{128, 256, 32, 4, 3, 1, 8, 5}, 1.99, 4.46, 0.317, 1.01, 0.456, 0.0429, 2.88, 0.91, 0, 0},
+    {{128, 128, 32, 4, 4, 1, 8, 5}, 1.68, 3.28, 0.259, 0.965, 0.239, 0.0169, 2.88, 1.46, 0, 0},
+    {{64, 128, 64, 4, 4, 1, 8, 5}, 1.06, 3.31, 0.339, 0.886, 0.175, 0.0204, 2.44, 1.81, 0, 0},
+    {{64, 64, 64, 4, 4, 1, 8, 5}, 1.49, 2.46, 0.277, 0.89, 0.184, 0.0205, 2.4, 1.89, 0, 0},
+    {{256, 256, 32, 4, 3, 1, 8, 13}, 1.42, 9.24, 0.363, 0.947, 0.827, 0.0445, 1.08, 1.01, 1.84, 0.984},
+    {{256, 128, 64, 4, 3, 1, 8, 13}, 2.17, 5.94, 0.545, 0.973, 0.525, 0.0163, 2.51, 0.81, 3.43, 0.868},
+    {{128, 128, 64, 4, 3, 1, 8, 13}, 2.41, 2.4, 0.345, 1.09, 0.422, 0.033, 3.78, 0.608, 4.52, 0.606},
+    {{64, 128, 64, 4, 4, 1, 8, 13}, 2.47, 1.72, 0.275, 0.991, 0.3, 0.0189, 2.52, 1.04, 5.37, 0.579},
+    {{128, 256, 32, 4, 3, 1, 8, 15}, 2.02, 4.34, 0.289, 1.04, 0.464, 0.0439, 0, 0, 3.05, 0.491},
+    {{128, 128, 32, 4, 4, 1, 8, 15}, 2.15, 2.5, 0.198, 1.09, 0.327, 0.0296, 0, 0, 3.36, 0.526},
+};
+const Timed kNoGammaTimed[] = {
+    {{128, 512, 32, 8, 3, 1, 8, 4}, 1.29, 5.59, 0.455, 1.03, 0.593, 0.079, 1.78, 1.02, 0, 0},
+    {{128, 256, 32, 4, 3, 1, 8, 5}, 2.96, 2.78, 0.302, 0.929, 0.417, 0.0607, 3.39, 0.7, 0, 0},
+    {{128, 128, 32, 4, 4, 1, 8, 5}, 2.56, 1.86, 0.237, 0.831, 0.281, 0.0185, 3.27, 1.16, 0, 0},
+    {{64, 128, 64, 4, 4, 1, 8, 5}, 1.76, 2.21, 0.31, 0.985, 0.205, 0.0199, 2.89, 1.48, 0, 0},
+    {{64, 64, 64, 4, 4, 1, 8, 5}, 2.13, 1.28, 0.248, 0.67, 0.125, 0.0229, 2.89, 1.23, 0, 0},
+    {{64, 128, 64, 4, 4, 1, 8, 14}, 1.88, 1.72, 0.27, 1.03, 0.377, 0.0233, 0, 0, 0, 0},
+    {{64, 64, 64, 4, 4, 1, 8, 14}, 2.43, 0.772, 0.183, 0.831, 0.394, 0.0171, 0, 0, 0, 0},
+    {{128, 128, 32, 4, 4, 1, 8, 16}, 2.31, 1.66, 0.193, 0.933, 0.356, 0.027, 0, 0, 0, 0},
+};
+const Timed kLhsTTimed[] = {
+    {{256, 256, 32, 4, 3, 1, 8, 1}, 1.06, 6.57, 0.364, 0.998, 0.739, 0.0383, 1.19, 0.962, 0, 0},
+    {{256, 128, 32, 4, 3, 1, 8, 1}, 2.7, 2.26, 0.218, 0.961, 0.709, 0.0227, 3.58, 0.718, 0, 0},
+    {{128, 256, 32, 4, 3, 1, 8, 1}, 2.57, 2.39, 0.21, 0.947, 0.77, 0.0321, 3.65, 0.689, 0, 0},
+    {{128, 128, 32, 4, 4, 1, 8, 1}, 2.12, 1.38, 0.164, 0.959, 0.386, 0.0106, 2.92, 1.29, 0, 0},
+    {{64, 256, 64, 4, 3, 1, 8, 1}, 1.67, 2.44, 0.367, 0.975, 0.529, 0.0123, 2.89, 1.19, 0, 0},
+    {{128, 64, 64, 4, 4, 1, 8, 1}, 1.25, 2.11, 0.26, 0.817, 0.378, 0.0145, 2.1, 1.82, 0, 0},
+    {{64, 128, 64, 4, 4, 1, 8, 1}, 1.25, 2.1, 0.254, 0.833, 0.407, 0.0145, 2.2, 1.71, 0, 0},
+    {{64, 64, 64, 4, 4, 1, 8, 1}, 2.1, 1.04, 0.189, 0.674, 0.325, 0.0343, 1.67, 1.92, 0, 0},
+    {{32, 128, 64, 4, 4, 1, 8, 1}, 1.46, 1.47, 0.209, 0.59, 0.489, 0.0212, 1.63, 2, 0, 0},
+};
+const Timed kLhsTimed[] = {
+    {{256, 256, 32, 8, 3, 1, 8, 0}, 1.21, 5.05, 0.412, 0.952, 0.852, 0.0519, 1.94, 1.01, 0, 0},
+    {{256, 128, 64, 8, 3, 1, 8, 0}, 1.25, 3.15, 0.589, 0.983, 0.549, 0.0173, 3, 1.03, 0, 0},
+    {{128, 256, 64, 4, 3, 1, 8, 0}, 1.53, 3.81, 0.661, 0.966, 0.419, 0.0274, 2.63, 0.91, 0, 0},
+    {{128, 128, 64, 4, 3, 1, 8, 0}, 1.9, 1.92, 0.354, 1.05, 0.436, 0.0138, 2.68, 1.32, 0, 0},
+    {{64, 256, 64, 4, 3, 1, 8, 0}, 2.05, 2.04, 0.368, 1.08, 0.482, 0.0158, 2.69, 1.26, 0, 0},
+    {{64, 128, 64, 4, 4, 1, 8, 0}, 1.16, 2.05, 0.247, 0.873, 0.441, 0.0161, 2.34, 1.7, 0, 0},
+    {{64, 64, 64, 4, 4, 1, 8, 0}, 1.83, 1.02, 0.183, 0.698, 0.47, 0.0196, 2.37, 1.51, 0, 0},
+    {{32, 128, 64, 4, 4, 1, 8, 0}, 2.03, 1.06, 0.188, 0.727, 0.448, 0.019, 2.31, 1.6, 0, 0},
+    {{256, 256, 32, 8, 3, 1, 8, 1}, 1.15, 5.73, 0.394, 0.963, 0.745, 0.0249, 0, 0, 0, 0},
+    {{128, 256, 32, 4, 3, 1, 8, 1}, 2.27, 2.29, 0.287, 0.994, 0.331, 0.0646, 0, 0, 0, 0},
+    {{128, 128, 32, 4, 4, 1, 8, 1}, 2.12, 1.29, 0.171, 0.954, 0.507, 0.0274, 0, 0, 0, 0},
+};
+
+// M <= 128 with a weight of at most 7 MiB, and (lhs.rhs, non-temporal blocks
+// only) of 7 to 28 MiB: the same fits to 160 shapes of each kind (120 for
+// the last), the weight warm in the caches as a call repeated over a few
+// layers leaves it.
+const Timed kFusedSkinnyTimed[] = {
+    {{64, 128, 64, 4, 4, 1, 8, 5}, 2.01, 1.98, 0.33, 0.878, 0.376, 0.0171, 2.31, 2.51, 0, 0},
+    {{64, 64, 64, 4, 4, 1, 8, 5}, 1.95, 1.83, 0.269, 0.921, 0.247, 0.0153, 2.43, 2.08, 0, 0},
+    {{32, 128, 64, 4, 4, 1, 8, 5}, 1.78, 1.81, 0.248, 0.929, 0.399, 0.0169, 2.64, 1.84, 0, 0},
+    {{128, 128, 64, 4, 3, 1, 8, 11}, 2.23, 2.23, 0.546, 0.9, 0.446, 0.0216, 1.97, 2.83, 0, 0},
+    {{64, 128, 64, 4, 3, 1, 8, 11}, 1.93, 1.87, 0.332, 0.856, 0.939, 0.0273, 2.47, 2.37, 0, 0},
+    {{32, 128, 128, 4, 3, 1, 8, 11}, 1.83, 1.87, 0.56, 0.939, 0.368, 0.173, 2.59, 2.14, 0, 0},
+    {{32, 128, 64, 4, 3, 1, 8, 11}, 1.82, 1.69, 0.255, 0.839, 0.761, 0.0822, 2.68, 1.69, 0, 0},
+    {{32, 128, 64, 4, 4, 1, 8, 12}, 1.82, 1.78, 0.263, 0.898, 0.481, 0.111, 2.68, 1.9, 0, 0},
+};
+const Timed kLhsTSkinnyTimed[] = {
+    {{64, 128, 64, 4, 4, 1, 8, 1}, 1.82, 1.81, 0.172, 0.896, 0.391, 0.0164, 2.79, 1.46, 0, 0},
+    {{64, 64, 64, 4, 4, 1, 8, 1}, 2.3, 1.42, 0.108, 0.428, 0.186, 0.0104, 2.82, 0.942, 0, 0},
+    {{32, 128, 64, 4, 4, 1, 8, 1}, 2.17, 1.51, 0.114, 0.551, 0.374, 0.0183, 2.93, 0.964, 0, 0},
+    {{128, 256, 32, 4, 3, 1, 8, 3}, 2.12, 2.12, 0.229, 0.9, 0.621, 0.0323, 1.89, 3.01, 0, 0},
+    {{128, 128, 32, 4, 4, 1, 8, 3}, 1.78, 1.78, 0.113, 0.9, 0.442, 0.0254, 2.83, 1.94, 0, 0},
+    {{64, 256, 64, 4, 3, 1, 8, 3}, 1.86, 1.86, 0.356, 0.9, 1.55, 0.0308, 2.5, 2.84, 0, 0},
+    {{64, 128, 64, 4, 4, 1, 8, 3}, 1.78, 1.73, 0.177, 0.858, 0.847, 0.0247, 2.97, 2.08, 0, 0},
+    {{32, 256, 64, 4, 4, 1, 8, 3}, 1.82, 1.82, 0.28, 0.9, 0.441, 0.133, 2.67, 2.2, 0, 0},
+    {{64, 64, 64, 4, 4, 1, 8, 3}, 2.16, 1.46, 0.119, 0.536, 0.389, 0.0198, 3.04, 1.1, 0, 0},
+    {{32, 128, 64, 4, 4, 1, 8, 3}, 2.07, 1.57, 0.117, 0.576, 0.531, 0.0437, 3.02, 1.58, 0, 0},
+};
+const Timed kLhsSkinnyTimed[] = {
+    {{64, 128, 64, 4, 4, 1, 8, 0}, 1.91, 1.91, 0.162, 0.9, 0.329, 0.0153, 2.59, 1.66, 0, 0},
+    {{64, 64, 64, 4, 4, 1, 8, 0}, 2.54, 1.42, 0.104, 0.268, 0.245, 0.0135, 2.7, 1.08, 0, 0},
+    {{32, 128, 128, 4, 3, 1, 8, 0}, 1.88, 1.79, 0.354, 0.833, 0.211, 0.017, 2.62, 1.45, 0, 0},
+    {{32, 128, 64, 4, 4, 1, 8, 0}, 2.4, 1.51, 0.121, 0.399, 0.242, 0.0153, 2.67, 1.13, 0, 0},
+    {{128, 128, 64, 4, 3, 1, 8, 2}, 1.96, 1.96, 0.259, 0.9, 0.387, 0.0204, 2.44, 2.48, 0, 0},
+    {{64, 128, 128, 4, 3, 1, 8, 2}, 1.83, 1.83, 0.433, 0.9, 0.628, 0.0283, 2.72, 2.35, 0, 0},
+    {{64, 128, 64, 4, 4, 1, 8, 2}, 1.91, 1.91, 0.153, 0.9, 0.469, 0.0282, 2.75, 1.88, 0, 0},
+};
+const Timed kLhsSkinnyStreamTimed[] = {
+    {{256, 128, 64, 8, 3, 1, 8, 2}, 2.15, 2.05, 0.596, 0.839, 0.172, 0.015, 1.32, 2.91, 0, 0},
+    {{128, 128, 64, 4, 3, 1, 8, 2}, 1.64, 1.58, 0.525, 0.749, 0.156, 0.0155, 1.47, 3.18, 0, 0},
+    {{64, 128, 128, 4, 3, 1, 8, 2}, 1.5, 1.56, 0.851, 0.943, 0.19, 0.0465, 2.42, 2.85, 0, 0},
+    {{64, 128, 64, 4, 4, 1, 8, 2}, 1.43, 1.42, 0.456, 0.78, 0.255, 0.0195, 2.07, 3.02, 0, 0},
+    {{32, 256, 64, 4, 4, 1, 8, 2}, 1.52, 1.62, 0.626, 0.936, 0.161, 0.0649, 2.82, 2.11, 0, 0},
+    {{64, 64, 64, 4, 4, 1, 8, 2}, 2.12, 0.629, 0.31, 0.708, 0.281, 0.0158, 1.71, 4.12, 0, 0},
+    {{32, 128, 128, 4, 3, 1, 8, 2}, 1.46, 1.6, 0.722, 0.962, 0.14, 0.0632, 2.83, 2.06, 0, 0},
+    {{32, 128, 64, 4, 4, 1, 8, 2}, 1.87, 0.956, 0.387, 0.867, 0.13, 0.048, 2.46, 2.37, 0, 0},
+};
+
+double fitted_time(const Timed& e, int parts, int M, int N, int K) {
+  const long long wgs = tiles_of(M, N, e.c.block_m, e.c.block_n) * parts;
+  const double n = (double)((wgs + kCUs - 1) / kCUs), f = wgs < kCUs ? (double)wgs / kCUs : 1.0;
+  const long long kt = ((long long)K + e.c.block_k - 1) / e.c.block_k;
+  const double L = (double)((kt + parts - 1) / parts), mn = (double)M * N * 1e-6;
+  double t = e.start + (e.tile + e.step * L * (1.0 + e.crowd * f)) * (1.0 + (n - 1.0) * e.more) +
+             e.read_mb * ((double)M + N) * K * 2e-6;
+  if (parts > 1) t += e.split + e.split_mb * parts * mn;
+  return t + e.pack + e.pack_mb * (double)M * K * 1e-6;
+}
+
+const Timed* timed(const Timed* table, int n, const mi_tile_cfg& c) {
+  for (int i = 0; i < n; ++i) {
+    const mi_tile_cfg& t = table[i].c;
+    if (t.block_m == c.block_m && t.block_n == c.block_n && t.block_k == c.block_k && t.waves == c.waves &&
+        t.lds_stages == c.lds_stages && t.variant == c.variant)
+      return &table[i];
+  }
+  return nullptr;
+}
+
+// Whether the call can run `c` in `parts` parts: at most one workgroup per
+// CU where K is split, no part empty, gamma of a part within the entries the
+// instance stages, and the workspace within its limit.  A split in parts
+// that are no power of two keeps at least 2688 of K in each.
+bool runs_split(int kernel_id, const mi_tile_cfg& c, int parts, int M, int N, int K) {
+  const long long kt = ((long long)K + c.block_k - 1) / c.block_k, kts = (kt + parts - 1) / parts;
+  if (parts > 1) {
+    if (!splittable(kernel_id, c.variant) || tiles_of(M, N, c.block_m, c.block_n) * parts > kCUs ||
+        (parts - 1) * kts >= kt || ((parts & (parts - 1)) != 0 && K < 2688LL * parts))
+      return false;
+  }
+  const mi::MiEntry* e = find(kernel_id, c);
+  if (!e || (e->gamma_kmax > 0 && kts * c.block_k > e->gamma_kmax)) return false;
+  mi_tile_cfg p = c;
+  p.split_k = parts;
+  return mi::workspace_bytes(kernel_id, p, M, N, K, kDefaultCus) <= kMaxWorkspace;
+}
+
+// `pick` (what the rules above choose), or the candidate of `table` with the
+// least fitted time where that is under `margin` of the pick's own fitted
+// time.  A pick that was not timed stays, and so does every pick of a call
+// past the timed range.
+mi_tile_cfg refined(int kernel_id, const Timed* table, int n, const mi_tile_cfg& pick, double margin, double max_flops,
+                    int M, int N, int K) {
+  const Timed* old = timed(table, n, pick);
+  if (!old || 2.0 * M * N * K > max_flops) return pick;
+  double best_t = margin * fitted_time(*old, pick.split_k, M, N, K);
+  mi_tile_cfg best = pick;
+  for (int i = 0; i < n; ++i) {
+    for (const int parts : {1, 2, 3, 4, 5, 6, 7, 8, 12, 16}) {
+      const double t = fitted_time(table[i], parts, M, N, K);
+      if (t < best_t && runs_split(kernel_id, table[i].c, parts, M, N, K)) {
+        best_t = t;
+        best = table[i].c;
+        best.split_k = parts;
+      }
+    }
+  }
+  return best;
+}
+
 // fp32: the MFMA kernel with K split over the waves (variant 3; variants 0,
 // in sequential K order, and 1 stay selectable), in the block and wave count
 // of the least estimated time (us).  The busiest CU runs `rounds` blocks.
@@ -464,6 +642,72 @@ mi_tile_cfg f32_default(int M, int N, int K) {
   return best;
 }
 
+template <int N>
+constexpr int count(const Timed (&)[N]) {
+  return N;
+}
+
+// Skinny M with a small weight.  A weight of up to 7 MiB is read through the
+// caches: the non-temporal blocks run it 1.1-1.3 x slower while the caches
+// hold it, and no faster when they do not (48x5504x704 fused, 7.8 MB: 7.1
+// against 8.4 us warm, 11.4 against 11.2 cold; 33 MB: 19.5 against 14.0
+// cold, so a larger one streams).  lhs.rhs also had no 32- and 64-row block
+// with a ring of 4: the refined pick runs within 1.025 of the fastest over
+// 160 shapes, the rules' own within 1.22 (1.012 against 1.14 at 7 to 28 MiB,
+// which keeps to non-temporal blocks); the fused kernel 1.014 against 1.074,
+// lhsT.rhs 1.027 against 1.082.
+constexpr long long kCachedWeight = 7LL << 20, kLhsSmallWeight = 28LL << 20;
+
+mi_tile_cfg refined_skinny(int kernel_id, int M, int N, int K) {
+  const long long weight = (long long)K * N * 2;
+  constexpr double kMargin = 0.95, kMaxFlops = 4e11;
+  if (kernel_id == MI_KERNEL_RMSNORM_MATMUL_BF16) {
+    const mi_tile_cfg pick = fused_default(M, N, K);
+    return weight > kCachedWeight ? pick
+                                  : refined(kernel_id, kFusedSkinnyTimed, count(kFusedSkinnyTimed), pick, kMargin,
+                                            kMaxFlops, M, N, K);
+  }
+  const bool lhs = kernel_id == MI_KERNEL_MATMUL_LHS_RHS_BF16;
+  const mi_tile_cfg pick = skinny_matmul_default(lhs, M, N, K);
+  if (weight > (lhs ? kLhsSmallWeight : kCachedWeight)) return pick;
+  if (!lhs) return refined(kernel_id, kLhsTSkinnyTimed, count(kLhsTSkinnyTimed), pick, kMargin, kMaxFlops, M, N, K);
+  if (weight > kCachedWeight)
+    return refined(kernel_id, kLhsSkinnyStreamTimed, count(kLhsSkinnyStreamTimed), pick, kMargin, kMaxFlops, M, N, K);
+  return refined(kernel_id, kLhsSkinnyTimed, count(kLhsSkinnyTimed), pick, kMargin, kMaxFlops, M, N, K);
+}
+
+// Either matmul past skinny M.  At 24 shapes of each drawn afterwards and
+// timed with every block and split the refined pick ran within 1.042
+// (lhsT.rhs) and 1.030 (lhs.rhs) of the fastest on average; over the first
+// campaign the rules' own ran within 1.06 and 1.05.  Its gains are splits of
+// 256-long blocks where the rules take a smaller block unsplit
+// (4736x1128x11552: 163 -> 130 us), and splits in 3 or 6 parts
+// (456x4232x6088 lhs.rhs: 49 -> 39 us).  256 x 128 in 2 parts stays: it is a
+// rule for shapes timed on their own.
+mi_tile_cfg refined_matmul(int kernel_id, bool lhs, int M, int N, int K) {
+  const mi_tile_cfg pick = matmul_default(kernel_id, lhs, M, N, K);
+  constexpr double kMaxFlops = 4e11;
+  if (!lhs) return refined(kernel_id, kLhsTTimed, count(kLhsTTimed), pick, 0.91, kMaxFlops, M, N, K);
+  if (pick.block_m == 256 && pick.block_n == 128 && pick.split_k == 2) return pick;
+  return refined(kernel_id, kLhsTimed, count(kLhsTimed), pick, 0.97, kMaxFlops, M, N, K);
+}
+
+// The fused kernel past skinny M.  The blocks that the rules above do not
+// know are the cached 64 x 64, 64 x 128 and 128 x 128 ones with a ring of 4
+// K tiles for W and 3 for x (rms_bf16_xreg.hip): at 50 shapes drawn
+// afterwards and timed with every block and split the refined pick ran
+// within 1.035 of the fastest on average; the rules' own ran within 1.18 at
+// 70 (600x304x584: 11.0 -> 6.6 us; 1176x1432x1168: 19.5 -> 12.8;
+// 6272x240x968: 19.9 -> 11.5).  Where M >= 256, N >= 2048 and K >= 2048 it
+// has to win by 30 %: tests fix the rules' picks at several shapes there
+// (all but 256x2048x2048, where 64 x 64 blocks take 13 us against 18.7, are
+// within 1.04 of the fastest).
+mi_tile_cfg refined_fused(int M, int N, int K) {
+  const double margin = M >= 256 && N >= 2048 && K >= 2048 ? 0.7 : 0.95;
+  return refined(MI_KERNEL_RMSNORM_MATMUL_BF16, kFusedTimed, count(kFusedTimed), fused_default(M, N, K), margin, 1.5e11,
+                 M, N, K);
+}
+
 }  // namespace
 
 // The library default: the estimates and rules above, fitted to timed
@@ -476,10 +720,10 @@ int pick_default(int kernel_id, int M, int N, int K, mi_tile_cfg* cfg) {
       break;
     case MI_KERNEL_MATMUL_LHST_RHS_BF16:
     case MI_KERNEL_MATMUL_LHS_RHS_BF16:
-      *cfg = M <= 128 ? skinny_matmul_default(lhs, M, N, K) : matmul_default(kernel_id, lhs, M, N, K);
+      *cfg = M <= 128 ? refined_skinny(kernel_id, M, N, K) : refined_matmul(kernel_id, lhs, M, N, K);
       break;
     case MI_KERNEL_RMSNORM_MATMUL_BF16:
-      *cfg = fused_default(M, N, K);
+      *cfg = M <= 128 ? refined_skinny(kernel_id, M, N, K) : refined_fused(M, N, K);
       break;
     default:
       *cfg = {256, 256, 64, 8, 2, 1, 8, 0};
@@ -489,44 +733,47 @@ int pick_default(int kernel_id, int M, int N, int K, mi_tile_cfg* cfg) {
 }
 
 // The fused kernel's default for a call without gamma: pick_default's
-// choice, except that its 128x128, 64x128 and 64x64 blocks (shapes of one
-// or two rounds of tiles, split or not) go to a gamma-free variant, unsplit:
-// 64x128 and 64x64 to variant 14 with the same block, 128x128 as below.
-// Variant 14 measured in interleaved rounds against
-// the default (no gamma): 0.60 x its time at 1024^3 (against the 4-part
-// split), 0.89 x at 2048^3, 0.90 x at 1024x4096x4096, 0.80 x at
-// 512x4096x4096, 0.78 x at 256x8192x2048; variant 16 at 128x128, against
-// variant 14's 128x128 block: 0.924-0.957 x (median 0.938) at twelve shapes
-// from 256x512x2048 to 4096x512x1024, with bitwise equal outputs.  The
-// larger blocks (128x512, 256x256 two-pass, 128x256) stay,
-// variant 14 being 0-8 % slower there.  Skinny M keeps its non-temporal
-// variants.
+// choice, except that its 128x128, 64x128 and 64x64 blocks (split or not) at
+// M > 128 give way to a gamma-free variant, unsplit, where that is faster by
+// the fitted times: 64x128 and 64x64 to variant 14 with the same block,
+// 128x128 to variant 16 at 128x128 or variant 14 at 64x128 or 64x64.  At 50
+// shapes drawn afterwards the pick ran within 1.036 of the fastest on
+// average, against 1.16 at 40 for always taking the gamma-free variant (152x160x5112, where 64x64 blocks unsplit leave 247 CUs idle: 23.3 ->
+// 9 us in 16 parts; 872x280x9560: 45 -> 21 us).  A pick that was not timed
+// without gamma moves as those rules did: a 128 x 128 block to the largest
+// block whose grid keeps more than half the CUs busy.  Measured without
+// gamma (us, 128 x 128 v16 / 64 x 128 v14 / 64 x 64 v14): 59.9 / 76.1 / 75.5
+// at 384x8192x8192 (192 tiles of 128 x 128); 29.2 / 23.5 / 28.7 at
+// 512x4096x4096 (128 tiles); 10.1 / 7.9 / 6.4 at 1024^3 (64 tiles).  The
+// larger blocks (128x512, 256x256 two-pass, 128x256) stay, variant 14 being
+// 0-8 % slower there.  Skinny M keeps its non-temporal variants.
 int pick_default_no_gamma(int M, int N, int K, mi_tile_cfg* cfg) {
   const int rc = pick_default(MI_KERNEL_RMSNORM_MATMUL_BF16, M, N, K, cfg);
   if (rc != MI_OK) return rc;
   const int v = cfg->variant, bm = cfg->block_m, bn = cfg->block_n;
   const bool one_pass_or_two = v == 4 || v == 5 || v == 13 || v == 15;
   const bool small_block = (bm == 128 && bn == 128) || (bm == 64 && bn == 128) || (bm == 64 && bn == 64);
-  if (M > 128 && one_pass_or_two && small_block) {
-    // A 128 x 128 pick takes the largest block whose grid keeps more than
-    // half the CUs busy: variant 16 at 128 x 128, else variant 14 at 64 x 128,
-    // else at 64 x 64.  Measured without gamma (us, 128 x 128 v16 / 64 x 128
-    // v14 / 64 x 64 v14): 59.9 / 76.1 / 75.5 at 384x8192x8192 (192 tiles of
-    // 128 x 128); 29.2 / 23.5 / 28.7 at 512x4096x4096 (128 tiles), 53.7 /
-    // 42.8 / 54.6 at 512x4096x8192, 16.3 / 12.9 / 14.3 at 1024x2048x2048;
-    // 10.1 / 7.9 / 6.4 at 1024^3 (64 tiles), 27.2 / 20.8 / 16.4 at
-    // 1024x1024x4096, 15.7 / 11.2 / 8.2 at 256x512x2048.
-    if (bm == 128) {
-      const long long t128 = tiles_of(M, N, 128, 128);
-      if (2 * t128 > kCUs)
-        *cfg = {128, 128, 32, 4, 4, 1, cfg->group_m, 16};
-      else if (4 * t128 > kCUs)
-        *cfg = {64, 128, 64, 4, 4, 1, cfg->group_m, 14};
-      else
-        *cfg = {64, 64, 64, 4, 4, 1, cfg->group_m, 14};
-    } else {
-      *cfg = {bm, bn, 64, 4, 4, 1, cfg->group_m, 14};
+  if (M <= 128 || !one_pass_or_two || !small_block) return MI_OK;
+  const mi_tile_cfg free[] = {{128, 128, 32, 4, 4, 1, 8, 16}, {64, 128, 64, 4, 4, 1, 8, 14}, {64, 64, 64, 4, 4, 1, 8, 14}};
+  const long long t128 = tiles_of(M, N, 128, 128);
+  int pick = bm == 128 ? (2 * t128 > kCUs ? 0 : 4 * t128 > kCUs ? 1 : 2) : bn == 128 ? 1 : 2;
+  const Timed* old = timed(kNoGammaTimed, count(kNoGammaTimed), *cfg);
+  if (old) {
+    double best_t = fitted_time(*old, cfg->split_k, M, N, K);
+    pick = -1;
+    for (int i = 0; i < 3; ++i) {
+      if (bm != 128 && (free[i].block_m != bm || free[i].block_n != bn)) continue;
+      const double t = fitted_time(*timed(kNoGammaTimed, count(kNoGammaTimed), free[i]), 1, M, N, K);
+      if (t < best_t) {
+        best_t = t;
+        pick = i;
+      }
     }
+  }
+  if (pick >= 0) {
+    const int group_m = cfg->group_m;
+    *cfg = free[pick];
+    cfg->group_m = group_m;
   }
   return MI_OK;
 }

@@ -47,6 +47,8 @@
   X(128, 128, 32, 4, 4)
 
 #define MI_LHS_SKINNY_CONFIGS(X) \
+  X(32, 128, 64, 4, 4)           \
+  X(64, 64, 64, 4, 4)            \
   X(32, 128, 128, 4, 3)          \
   X(32, 256, 64, 4, 4)           \
   X(64, 128, 64, 4, 4)           \
