@@ -427,73 +427,75 @@ mi_tile_cfg fused_default(int M, int N, int K) {
 }
 
 // Fitted times.  A candidate's time (us) at a shape is
-//   start + (tile + step * L * (1 + crowd * f)) * (1 + (n - 1) * more)
+//   start + (tile + step * L * (1 + crowd * f * (1 + drift * L * block_k / 1e4)))
+//         * (1 + (n - 1) * more)
 //   + read_mb * (the inputs' MB)
 //   [+ split + split_mb * p * M * N / 1e6]      K split in p parts
 //   [+ pack + pack_mb * M * K / 1e6]            the two-pass fused kernels
 // with L the K tiles of a part, n the workgroups of the busiest CU, and f
 // the share of CUs that have one (at most 1): one tile's fixed cost, its cost
-// per K tile (more when every CU loads at once), and the further tiles of a
-// CU, which overlap the first one's loads.  The coefficients are fitted to
+// per K tile (more when every CU loads at once, and more the longer K is, as
+// workgroups that share panels drift apart), and the further tiles of a CU,
+// which overlap the first one's loads.  The coefficients are fitted to
 // every candidate block in 1-8, 12 and 16 parts, timed at 480 fused, 320
 // no-gamma, 380 lhsT.rhs and 380 lhs.rhs shapes with M > 128 (sizes spread
 // over their logarithm, N up to 28672, K up to 16384), three sets of inputs
 // in turn.  Fitted without half of the second campaigns' shapes, the least
-// fitted time is within 1.012, 1.023, 1.022 and 1.021 of the fastest on
+// fitted time is within 1.013, 1.020, 1.022 and 1.017 of the fastest on
 // average at those.
 struct Timed {
   mi_tile_cfg c;
-  double start, tile, step, more, crowd, read_mb, split, split_mb, pack, pack_mb;
+  double start, tile, step, more, crowd, drift, read_mb, split, split_mb, pack, pack_mb;
 };
 
 const Timed kFusedTimed[] = {
-    {{128, 512, 32, 8, 3, 1, 8, 4}, 1.39, 5.75, 0.444, 1.04, 0.744, 0.0336, 2.4, 1.06, 0, 0},
-    {{128, 128, 64, 4, 2, 1, 8, 4}, 1.78, 3.33, 0.525, 0.933, 0.26, 0.0192, 2.86, 1.32, 0, 0},
-    {{256, 128, 32, 8, 3, 1, 8, 5}, 1.83, 3.93, 0.375, 1.05, 0.468, 0.0166, 3.92, 1.04, 0, 0},
-    {{128, 256, 32, 4, 3, 1, 8, 5}, 1.99, 4.46, 0.317, 1.01, 0.456, 0.0429, 2.88, 0.91, 0, 0},
-    {{128, 128, 32, 4, 4, 1, 8, 5}, 1.68, 3.28, 0.259, 0.965, 0.239, 0.0169, 2.88, 1.46, 0, 0},
-    {{64, 128, 64, 4, 4, 1, 8, 5}, 1.06, 3.31, 0.339, 0.886, 0.175, 0.0204, 2.44, 1.81, 0, 0},
-    {{64, 64, 64, 4, 4, 1, 8, 5}, 1.49, 2.46, 0.277, 0.89, 0.184, 0.0205, 2.4, 1.89, 0, 0},
-    {{256, 256, 32, 4, 3, 1, 8, 13}, 1.42, 9.24, 0.363, 0.947, 0.827, 0.0445, 1.08, 1.01, 1.84, 0.984},
-    {{256, 128, 64, 4, 3, 1, 8, 13}, 2.17, 5.94, 0.545, 0.973, 0.525, 0.0163, 2.51, 0.81, 3.43, 0.868},
-    {{128, 128, 64, 4, 3, 1, 8, 13}, 2.41, 2.4, 0.345, 1.09, 0.422, 0.033, 3.78, 0.608, 4.52, 0.606},
-    {{64, 128, 64, 4, 4, 1, 8, 13}, 2.47, 1.72, 0.275, 0.991, 0.3, 0.0189, 2.52, 1.04, 5.37, 0.579},
-    {{128, 256, 32, 4, 3, 1, 8, 15}, 2.02, 4.34, 0.289, 1.04, 0.464, 0.0439, 0, 0, 3.05, 0.491},
-    {{128, 128, 32, 4, 4, 1, 8, 15}, 2.15, 2.5, 0.198, 1.09, 0.327, 0.0296, 0, 0, 3.36, 0.526},
+    {{128, 512, 32, 8, 3, 1, 8, 4}, 1.28, 6.28, 0.434, 1.08, 0.54, 1.39, 0.0379, 2.2, 1.16, 0, 0},
+    {{128, 128, 64, 4, 2, 1, 8, 4}, 1.75, 3.4, 0.521, 0.932, 0.244, 0.317, 0.0192, 2.85, 1.34, 0, 0},
+    {{256, 128, 32, 8, 3, 1, 8, 5}, 1.76, 4.09, 0.369, 1.04, 0.444, 0.381, 0.017, 3.9, 1.07, 0, 0},
+    {{128, 256, 32, 4, 3, 1, 8, 5}, 1.79, 4.91, 0.304, 1.02, 0.354, 1.53, 0.0472, 2.83, 0.98, 0, 0},
+    {{128, 128, 32, 4, 4, 1, 8, 5}, 1.66, 3.33, 0.258, 0.966, 0.223, 0.307, 0.0171, 2.86, 1.48, 0, 0},
+    {{64, 128, 64, 4, 4, 1, 8, 5}, 1.06, 3.32, 0.34, 0.891, 0.153, 0.261, 0.0211, 2.43, 1.83, 0, 0},
+    {{64, 64, 64, 4, 4, 1, 8, 5}, 1.49, 2.47, 0.278, 0.895, 0.163, 0.252, 0.021, 2.39, 1.92, 0, 0},
+    {{256, 256, 32, 4, 3, 1, 8, 13}, 1.46, 9.27, 0.365, 0.968, 0.743, 0.187, 0.0465, 1.06, 1.03, 1.91, 0.98},
+    {{256, 128, 64, 4, 3, 1, 8, 13}, 2.16, 6.19, 0.544, 0.976, 0.471, 0.231, 0.017, 2.45, 0.843, 3.4, 0.861},
+    {{128, 128, 64, 4, 3, 1, 8, 13}, 2.39, 2.8, 0.324, 1.05, 0.418, 0.667, 0.0348, 3.79, 0.653, 4.35, 0.597},
+    {{64, 128, 64, 4, 4, 1, 8, 13}, 2.47, 1.79, 0.271, 0.992, 0.281, 0.297, 0.0194, 2.47, 1.07, 5.39, 0.58},
+    {{128, 256, 32, 4, 3, 1, 8, 15}, 1.99, 4.61, 0.287, 1.04, 0.412, 0.397, 0.0435, 0, 0, 2.99, 0.454},
+    {{128, 128, 32, 4, 4, 1, 8, 15}, 2.14, 2.73, 0.188, 1.07, 0.326, 0.557, 0.0301, 0, 0, 3.33, 0.496},
 };
 const Timed kNoGammaTimed[] = {
-    {{128, 512, 32, 8, 3, 1, 8, 4}, 1.29, 5.59, 0.455, 1.03, 0.593, 0.079, 1.78, 1.02, 0, 0},
-    {{128, 256, 32, 4, 3, 1, 8, 5}, 2.96, 2.78, 0.302, 0.929, 0.417, 0.0607, 3.39, 0.7, 0, 0},
-    {{128, 128, 32, 4, 4, 1, 8, 5}, 2.56, 1.86, 0.237, 0.831, 0.281, 0.0185, 3.27, 1.16, 0, 0},
-    {{64, 128, 64, 4, 4, 1, 8, 5}, 1.76, 2.21, 0.31, 0.985, 0.205, 0.0199, 2.89, 1.48, 0, 0},
-    {{64, 64, 64, 4, 4, 1, 8, 5}, 2.13, 1.28, 0.248, 0.67, 0.125, 0.0229, 2.89, 1.23, 0, 0},
-    {{64, 128, 64, 4, 4, 1, 8, 14}, 1.88, 1.72, 0.27, 1.03, 0.377, 0.0233, 0, 0, 0, 0},
-    {{64, 64, 64, 4, 4, 1, 8, 14}, 2.43, 0.772, 0.183, 0.831, 0.394, 0.0171, 0, 0, 0, 0},
-    {{128, 128, 32, 4, 4, 1, 8, 16}, 2.31, 1.66, 0.193, 0.933, 0.356, 0.027, 0, 0, 0, 0},
+    {{128, 512, 32, 8, 3, 1, 8, 4}, 1.16, 6.03, 0.438, 1.02, 0.554, 0.609, 0.0803, 1.72, 1.06, 0, 0},
+    {{128, 256, 32, 4, 3, 1, 8, 5}, 2.7, 3.62, 0.275, 0.886, 0.329, 2.32, 0.0621, 3.27, 0.796, 0, 0},
+    {{128, 128, 32, 4, 4, 1, 8, 5}, 2.56, 2.08, 0.223, 0.839, 0.224, 1.99, 0.0195, 3.35, 1.21, 0, 0},
+    {{64, 128, 64, 4, 4, 1, 8, 5}, 1.71, 2.27, 0.308, 0.983, 0.192, 0.316, 0.0203, 2.9, 1.5, 0, 0},
+    {{64, 64, 64, 4, 4, 1, 8, 5}, 2.13, 1.29, 0.246, 0.67, 0.121, 0.316, 0.0225, 2.89, 1.24, 0, 0},
+    {{64, 128, 64, 4, 4, 1, 8, 14}, 1.72, 1.94, 0.264, 1.03, 0.305, 0.617, 0.0291, 0, 0, 0, 0},
+    {{64, 64, 64, 4, 4, 1, 8, 14}, 2.41, 0.862, 0.178, 0.84, 0.326, 0.928, 0.0173, 0, 0, 0, 0},
+    {{128, 128, 32, 4, 4, 1, 8, 16}, 2.29, 1.8, 0.186, 0.945, 0.297, 0.843, 0.0271, 0, 0, 0, 0},
 };
 const Timed kLhsTTimed[] = {
-    {{256, 256, 32, 4, 3, 1, 8, 1}, 1.06, 6.57, 0.364, 0.998, 0.739, 0.0383, 1.19, 0.962, 0, 0},
-    {{256, 128, 32, 4, 3, 1, 8, 1}, 2.7, 2.26, 0.218, 0.961, 0.709, 0.0227, 3.58, 0.718, 0, 0},
-    {{128, 256, 32, 4, 3, 1, 8, 1}, 2.57, 2.39, 0.21, 0.947, 0.77, 0.0321, 3.65, 0.689, 0, 0},
-    {{128, 128, 32, 4, 4, 1, 8, 1}, 2.12, 1.38, 0.164, 0.959, 0.386, 0.0106, 2.92, 1.29, 0, 0},
-    {{64, 256, 64, 4, 3, 1, 8, 1}, 1.67, 2.44, 0.367, 0.975, 0.529, 0.0123, 2.89, 1.19, 0, 0},
-    {{128, 64, 64, 4, 4, 1, 8, 1}, 1.25, 2.11, 0.26, 0.817, 0.378, 0.0145, 2.1, 1.82, 0, 0},
-    {{64, 128, 64, 4, 4, 1, 8, 1}, 1.25, 2.1, 0.254, 0.833, 0.407, 0.0145, 2.2, 1.71, 0, 0},
-    {{64, 64, 64, 4, 4, 1, 8, 1}, 2.1, 1.04, 0.189, 0.674, 0.325, 0.0343, 1.67, 1.92, 0, 0},
-    {{32, 128, 64, 4, 4, 1, 8, 1}, 1.46, 1.47, 0.209, 0.59, 0.489, 0.0212, 1.63, 2, 0, 0},
+    {{256, 256, 32, 4, 3, 1, 8, 1}, 1.06, 6.87, 0.353, 1.02, 0.664, 0.425, 0.042, 1.17, 1, 0, 0},
+    {{256, 128, 32, 4, 3, 1, 8, 1}, 2.54, 2.66, 0.211, 0.968, 0.549, 1.03, 0.0265, 3.46, 0.818, 0, 0},
+    {{128, 256, 32, 4, 3, 1, 8, 1}, 2.46, 2.71, 0.204, 0.966, 0.595, 0.913, 0.0399, 3.53, 0.777, 0, 0},
+    {{128, 128, 32, 4, 4, 1, 8, 1}, 2.04, 1.54, 0.159, 0.955, 0.324, 1.06, 0.0113, 2.93, 1.32, 0, 0},
+    {{64, 256, 64, 4, 3, 1, 8, 1}, 1.54, 2.63, 0.362, 0.957, 0.496, 0.38, 0.0128, 2.88, 1.23, 0, 0},
+    {{128, 64, 64, 4, 4, 1, 8, 1}, 1.23, 2.14, 0.259, 0.818, 0.353, 0.264, 0.0148, 2.1, 1.84, 0, 0},
+    {{64, 128, 64, 4, 4, 1, 8, 1}, 1.23, 2.13, 0.253, 0.836, 0.376, 0.264, 0.0151, 2.2, 1.73, 0, 0},
+    {{64, 64, 64, 4, 4, 1, 8, 1}, 2.12, 1.04, 0.188, 0.68, 0.31, 0.295, 0.0325, 1.68, 1.93, 0, 0},
+    {{32, 128, 64, 4, 4, 1, 8, 1}, 1.48, 1.47, 0.207, 0.597, 0.463, 0.285, 0.021, 1.63, 2.03, 0, 0},
 };
 const Timed kLhsTimed[] = {
-    {{256, 256, 32, 8, 3, 1, 8, 0}, 1.21, 5.05, 0.412, 0.952, 0.852, 0.0519, 1.94, 1.01, 0, 0},
-    {{256, 128, 64, 8, 3, 1, 8, 0}, 1.25, 3.15, 0.589, 0.983, 0.549, 0.0173, 3, 1.03, 0, 0},
-    {{128, 256, 64, 4, 3, 1, 8, 0}, 1.53, 3.81, 0.661, 0.966, 0.419, 0.0274, 2.63, 0.91, 0, 0},
-    {{128, 128, 64, 4, 3, 1, 8, 0}, 1.9, 1.92, 0.354, 1.05, 0.436, 0.0138, 2.68, 1.32, 0, 0},
-    {{64, 256, 64, 4, 3, 1, 8, 0}, 2.05, 2.04, 0.368, 1.08, 0.482, 0.0158, 2.69, 1.26, 0, 0},
-    {{64, 128, 64, 4, 4, 1, 8, 0}, 1.16, 2.05, 0.247, 0.873, 0.441, 0.0161, 2.34, 1.7, 0, 0},
-    {{64, 64, 64, 4, 4, 1, 8, 0}, 1.83, 1.02, 0.183, 0.698, 0.47, 0.0196, 2.37, 1.51, 0, 0},
-    {{32, 128, 64, 4, 4, 1, 8, 0}, 2.03, 1.06, 0.188, 0.727, 0.448, 0.019, 2.31, 1.6, 0, 0},
-    {{256, 256, 32, 8, 3, 1, 8, 1}, 1.15, 5.73, 0.394, 0.963, 0.745, 0.0249, 0, 0, 0, 0},
-    {{128, 256, 32, 4, 3, 1, 8, 1}, 2.27, 2.29, 0.287, 0.994, 0.331, 0.0646, 0, 0, 0, 0},
-    {{128, 128, 32, 4, 4, 1, 8, 1}, 2.12, 1.29, 0.171, 0.954, 0.507, 0.0274, 0, 0, 0, 0},
+    {{256, 256, 32, 8, 3, 1, 8, 0}, 1.18, 5.45, 0.398, 0.974, 0.729, 0.641, 0.0557, 1.86, 1.08, 0, 0},
+    {{256, 128, 64, 8, 3, 1, 8, 0}, 1.1, 3.56, 0.568, 0.986, 0.454, 0.83, 0.0179, 2.9, 1.15, 0, 0},
+    {{128, 256, 64, 4, 3, 1, 8, 0}, 1.5, 4.06, 0.643, 0.977, 0.365, 0.48, 0.0303, 2.55, 0.986, 0, 0},
+    {{128, 128, 64, 4, 3, 1, 8, 0}, 1.68, 2.25, 0.343, 1.02, 0.377, 0.761, 0.0148, 2.65, 1.41, 0, 0},
+    {{64, 256, 64, 4, 3, 1, 8, 0}, 1.85, 2.34, 0.359, 1.05, 0.435, 0.56, 0.0167, 2.67, 1.32, 0, 0},
+    {{64, 128, 64, 4, 4, 1, 8, 0}, 1.11, 2.13, 0.245, 0.872, 0.395, 0.372, 0.0165, 2.32, 1.75, 0, 0},
+    {{64, 64, 64, 4, 4, 1, 8, 0}, 1.82, 1.07, 0.181, 0.698, 0.429, 0.45, 0.0197, 2.36, 1.57, 0, 0},
+    {{32, 128, 64, 4, 4, 1, 8, 0}, 2.04, 1.11, 0.183, 0.732, 0.403, 0.696, 0.0187, 2.32, 1.65, 0, 0},
+    {{256, 256, 32, 8, 3, 1, 8, 1}, 1.31, 5.87, 0.373, 0.988, 0.714, 0.387, 0.0274, 0, 0, 0, 0},
+    {{128, 256, 32, 4, 3, 1, 8, 1}, 2.4, 2.36, 0.277, 1.02, 0.286, 0.61, 0.0625, 0, 0, 0, 0},
+    {{128, 128, 32, 4, 4, 1, 8, 1}, 2.08, 1.41, 0.168, 0.955, 0.444, 0.407, 0.0282, 0, 0, 0, 0},
 };
 
 // M <= 128 with a weight of at most 7 MiB, and (lhs.rhs, non-temporal blocks
@@ -501,45 +503,45 @@ const Timed kLhsTimed[] = {
 // the last), the weight warm in the caches as a call repeated over a few
 // layers leaves it.
 const Timed kFusedSkinnyTimed[] = {
-    {{64, 128, 64, 4, 4, 1, 8, 5}, 2.01, 1.98, 0.33, 0.878, 0.376, 0.0171, 2.31, 2.51, 0, 0},
-    {{64, 64, 64, 4, 4, 1, 8, 5}, 1.95, 1.83, 0.269, 0.921, 0.247, 0.0153, 2.43, 2.08, 0, 0},
-    {{32, 128, 64, 4, 4, 1, 8, 5}, 1.78, 1.81, 0.248, 0.929, 0.399, 0.0169, 2.64, 1.84, 0, 0},
-    {{128, 128, 64, 4, 3, 1, 8, 11}, 2.23, 2.23, 0.546, 0.9, 0.446, 0.0216, 1.97, 2.83, 0, 0},
-    {{64, 128, 64, 4, 3, 1, 8, 11}, 1.93, 1.87, 0.332, 0.856, 0.939, 0.0273, 2.47, 2.37, 0, 0},
-    {{32, 128, 128, 4, 3, 1, 8, 11}, 1.83, 1.87, 0.56, 0.939, 0.368, 0.173, 2.59, 2.14, 0, 0},
-    {{32, 128, 64, 4, 3, 1, 8, 11}, 1.82, 1.69, 0.255, 0.839, 0.761, 0.0822, 2.68, 1.69, 0, 0},
-    {{32, 128, 64, 4, 4, 1, 8, 12}, 1.82, 1.78, 0.263, 0.898, 0.481, 0.111, 2.68, 1.9, 0, 0},
+    {{64, 128, 64, 4, 4, 1, 8, 5}, 2.01, 1.98, 0.33, 0.878, 0.376, 0, 0.0171, 2.31, 2.51, 0, 0},
+    {{64, 64, 64, 4, 4, 1, 8, 5}, 1.95, 1.83, 0.269, 0.921, 0.247, 0, 0.0153, 2.43, 2.08, 0, 0},
+    {{32, 128, 64, 4, 4, 1, 8, 5}, 1.78, 1.81, 0.248, 0.929, 0.399, 0, 0.0169, 2.64, 1.84, 0, 0},
+    {{128, 128, 64, 4, 3, 1, 8, 11}, 2.23, 2.23, 0.546, 0.9, 0.446, 0, 0.0216, 1.97, 2.83, 0, 0},
+    {{64, 128, 64, 4, 3, 1, 8, 11}, 1.93, 1.87, 0.332, 0.856, 0.939, 0, 0.0273, 2.47, 2.37, 0, 0},
+    {{32, 128, 128, 4, 3, 1, 8, 11}, 1.83, 1.87, 0.56, 0.939, 0.368, 0, 0.173, 2.59, 2.14, 0, 0},
+    {{32, 128, 64, 4, 3, 1, 8, 11}, 1.82, 1.69, 0.255, 0.839, 0.761, 0, 0.0822, 2.68, 1.69, 0, 0},
+    {{32, 128, 64, 4, 4, 1, 8, 12}, 1.82, 1.78, 0.263, 0.898, 0.481, 0, 0.111, 2.68, 1.9, 0, 0},
 };
 const Timed kLhsTSkinnyTimed[] = {
-    {{64, 128, 64, 4, 4, 1, 8, 1}, 1.82, 1.81, 0.172, 0.896, 0.391, 0.0164, 2.79, 1.46, 0, 0},
-    {{64, 64, 64, 4, 4, 1, 8, 1}, 2.3, 1.42, 0.108, 0.428, 0.186, 0.0104, 2.82, 0.942, 0, 0},
-    {{32, 128, 64, 4, 4, 1, 8, 1}, 2.17, 1.51, 0.114, 0.551, 0.374, 0.0183, 2.93, 0.964, 0, 0},
-    {{128, 256, 32, 4, 3, 1, 8, 3}, 2.12, 2.12, 0.229, 0.9, 0.621, 0.0323, 1.89, 3.01, 0, 0},
-    {{128, 128, 32, 4, 4, 1, 8, 3}, 1.78, 1.78, 0.113, 0.9, 0.442, 0.0254, 2.83, 1.94, 0, 0},
-    {{64, 256, 64, 4, 3, 1, 8, 3}, 1.86, 1.86, 0.356, 0.9, 1.55, 0.0308, 2.5, 2.84, 0, 0},
-    {{64, 128, 64, 4, 4, 1, 8, 3}, 1.78, 1.73, 0.177, 0.858, 0.847, 0.0247, 2.97, 2.08, 0, 0},
-    {{32, 256, 64, 4, 4, 1, 8, 3}, 1.82, 1.82, 0.28, 0.9, 0.441, 0.133, 2.67, 2.2, 0, 0},
-    {{64, 64, 64, 4, 4, 1, 8, 3}, 2.16, 1.46, 0.119, 0.536, 0.389, 0.0198, 3.04, 1.1, 0, 0},
-    {{32, 128, 64, 4, 4, 1, 8, 3}, 2.07, 1.57, 0.117, 0.576, 0.531, 0.0437, 3.02, 1.58, 0, 0},
+    {{64, 128, 64, 4, 4, 1, 8, 1}, 1.82, 1.81, 0.172, 0.896, 0.391, 0, 0.0164, 2.79, 1.46, 0, 0},
+    {{64, 64, 64, 4, 4, 1, 8, 1}, 2.3, 1.42, 0.108, 0.428, 0.186, 0, 0.0104, 2.82, 0.942, 0, 0},
+    {{32, 128, 64, 4, 4, 1, 8, 1}, 2.17, 1.51, 0.114, 0.551, 0.374, 0, 0.0183, 2.93, 0.964, 0, 0},
+    {{128, 256, 32, 4, 3, 1, 8, 3}, 2.12, 2.12, 0.229, 0.9, 0.621, 0, 0.0323, 1.89, 3.01, 0, 0},
+    {{128, 128, 32, 4, 4, 1, 8, 3}, 1.78, 1.78, 0.113, 0.9, 0.442, 0, 0.0254, 2.83, 1.94, 0, 0},
+    {{64, 256, 64, 4, 3, 1, 8, 3}, 1.86, 1.86, 0.356, 0.9, 1.55, 0, 0.0308, 2.5, 2.84, 0, 0},
+    {{64, 128, 64, 4, 4, 1, 8, 3}, 1.78, 1.73, 0.177, 0.858, 0.847, 0, 0.0247, 2.97, 2.08, 0, 0},
+    {{32, 256, 64, 4, 4, 1, 8, 3}, 1.82, 1.82, 0.28, 0.9, 0.441, 0, 0.133, 2.67, 2.2, 0, 0},
+    {{64, 64, 64, 4, 4, 1, 8, 3}, 2.16, 1.46, 0.119, 0.536, 0.389, 0, 0.0198, 3.04, 1.1, 0, 0},
+    {{32, 128, 64, 4, 4, 1, 8, 3}, 2.07, 1.57, 0.117, 0.576, 0.531, 0, 0.0437, 3.02, 1.58, 0, 0},
 };
 const Timed kLhsSkinnyTimed[] = {
-    {{64, 128, 64, 4, 4, 1, 8, 0}, 1.91, 1.91, 0.162, 0.9, 0.329, 0.0153, 2.59, 1.66, 0, 0},
-    {{64, 64, 64, 4, 4, 1, 8, 0}, 2.54, 1.42, 0.104, 0.268, 0.245, 0.0135, 2.7, 1.08, 0, 0},
-    {{32, 128, 128, 4, 3, 1, 8, 0}, 1.88, 1.79, 0.354, 0.833, 0.211, 0.017, 2.62, 1.45, 0, 0},
-    {{32, 128, 64, 4, 4, 1, 8, 0}, 2.4, 1.51, 0.121, 0.399, 0.242, 0.0153, 2.67, 1.13, 0, 0},
-    {{128, 128, 64, 4, 3, 1, 8, 2}, 1.96, 1.96, 0.259, 0.9, 0.387, 0.0204, 2.44, 2.48, 0, 0},
-    {{64, 128, 128, 4, 3, 1, 8, 2}, 1.83, 1.83, 0.433, 0.9, 0.628, 0.0283, 2.72, 2.35, 0, 0},
-    {{64, 128, 64, 4, 4, 1, 8, 2}, 1.91, 1.91, 0.153, 0.9, 0.469, 0.0282, 2.75, 1.88, 0, 0},
+    {{64, 128, 64, 4, 4, 1, 8, 0}, 1.91, 1.91, 0.162, 0.9, 0.329, 0, 0.0153, 2.59, 1.66, 0, 0},
+    {{64, 64, 64, 4, 4, 1, 8, 0}, 2.54, 1.42, 0.104, 0.268, 0.245, 0, 0.0135, 2.7, 1.08, 0, 0},
+    {{32, 128, 128, 4, 3, 1, 8, 0}, 1.88, 1.79, 0.354, 0.833, 0.211, 0, 0.017, 2.62, 1.45, 0, 0},
+    {{32, 128, 64, 4, 4, 1, 8, 0}, 2.4, 1.51, 0.121, 0.399, 0.242, 0, 0.0153, 2.67, 1.13, 0, 0},
+    {{128, 128, 64, 4, 3, 1, 8, 2}, 1.96, 1.96, 0.259, 0.9, 0.387, 0, 0.0204, 2.44, 2.48, 0, 0},
+    {{64, 128, 128, 4, 3, 1, 8, 2}, 1.83, 1.83, 0.433, 0.9, 0.628, 0, 0.0283, 2.72, 2.35, 0, 0},
+    {{64, 128, 64, 4, 4, 1, 8, 2}, 1.91, 1.91, 0.153, 0.9, 0.469, 0, 0.0282, 2.75, 1.88, 0, 0},
 };
 const Timed kLhsSkinnyStreamTimed[] = {
-    {{256, 128, 64, 8, 3, 1, 8, 2}, 2.15, 2.05, 0.596, 0.839, 0.172, 0.015, 1.32, 2.91, 0, 0},
-    {{128, 128, 64, 4, 3, 1, 8, 2}, 1.64, 1.58, 0.525, 0.749, 0.156, 0.0155, 1.47, 3.18, 0, 0},
-    {{64, 128, 128, 4, 3, 1, 8, 2}, 1.5, 1.56, 0.851, 0.943, 0.19, 0.0465, 2.42, 2.85, 0, 0},
-    {{64, 128, 64, 4, 4, 1, 8, 2}, 1.43, 1.42, 0.456, 0.78, 0.255, 0.0195, 2.07, 3.02, 0, 0},
-    {{32, 256, 64, 4, 4, 1, 8, 2}, 1.52, 1.62, 0.626, 0.936, 0.161, 0.0649, 2.82, 2.11, 0, 0},
-    {{64, 64, 64, 4, 4, 1, 8, 2}, 2.12, 0.629, 0.31, 0.708, 0.281, 0.0158, 1.71, 4.12, 0, 0},
-    {{32, 128, 128, 4, 3, 1, 8, 2}, 1.46, 1.6, 0.722, 0.962, 0.14, 0.0632, 2.83, 2.06, 0, 0},
-    {{32, 128, 64, 4, 4, 1, 8, 2}, 1.87, 0.956, 0.387, 0.867, 0.13, 0.048, 2.46, 2.37, 0, 0},
+    {{256, 128, 64, 8, 3, 1, 8, 2}, 2.15, 2.05, 0.596, 0.839, 0.172, 0, 0.015, 1.32, 2.91, 0, 0},
+    {{128, 128, 64, 4, 3, 1, 8, 2}, 1.64, 1.58, 0.525, 0.749, 0.156, 0, 0.0155, 1.47, 3.18, 0, 0},
+    {{64, 128, 128, 4, 3, 1, 8, 2}, 1.5, 1.56, 0.851, 0.943, 0.19, 0, 0.0465, 2.42, 2.85, 0, 0},
+    {{64, 128, 64, 4, 4, 1, 8, 2}, 1.43, 1.42, 0.456, 0.78, 0.255, 0, 0.0195, 2.07, 3.02, 0, 0},
+    {{32, 256, 64, 4, 4, 1, 8, 2}, 1.52, 1.62, 0.626, 0.936, 0.161, 0, 0.0649, 2.82, 2.11, 0, 0},
+    {{64, 64, 64, 4, 4, 1, 8, 2}, 2.12, 0.629, 0.31, 0.708, 0.281, 0, 0.0158, 1.71, 4.12, 0, 0},
+    {{32, 128, 128, 4, 3, 1, 8, 2}, 1.46, 1.6, 0.722, 0.962, 0.14, 0, 0.0632, 2.83, 2.06, 0, 0},
+    {{32, 128, 64, 4, 4, 1, 8, 2}, 1.87, 0.956, 0.387, 0.867, 0.13, 0, 0.048, 2.46, 2.37, 0, 0},
 };
 
 double fitted_time(const Timed& e, int parts, int M, int N, int K) {
@@ -547,7 +549,7 @@ double fitted_time(const Timed& e, int parts, int M, int N, int K) {
   const double n = (double)((wgs + kCUs - 1) / kCUs), f = wgs < kCUs ? (double)wgs / kCUs : 1.0;
   const long long kt = ((long long)K + e.c.block_k - 1) / e.c.block_k;
   const double L = (double)((kt + parts - 1) / parts), mn = (double)M * N * 1e-6;
-  double t = e.start + (e.tile + e.step * L * (1.0 + e.crowd * f)) * (1.0 + (n - 1.0) * e.more) +
+  double t = e.start + (e.tile + e.step * L * (1.0 + e.crowd * f * (1.0 + e.drift * L * e.c.block_k * 1e-4))) * (1.0 + (n - 1.0) * e.more) +
              e.read_mb * ((double)M + N) * K * 2e-6;
   if (parts > 1) t += e.split + e.split_mb * parts * mn;
   return t + e.pack + e.pack_mb * (double)M * K * 1e-6;
@@ -676,27 +678,27 @@ mi_tile_cfg refined_skinny(int kernel_id, int M, int N, int K) {
   return refined(kernel_id, kLhsSkinnyTimed, count(kLhsSkinnyTimed), pick, kMargin, kMaxFlops, M, N, K);
 }
 
-// Either matmul past skinny M.  At 24 shapes of each drawn afterwards and
-// timed with every block and split the refined pick ran within 1.042
-// (lhsT.rhs) and 1.030 (lhs.rhs) of the fastest on average; over the first
+// Either matmul past skinny M.  At 30 shapes of each drawn afterwards and
+// timed with every block and split the refined pick ran within 1.030
+// (lhsT.rhs) and 1.028 (lhs.rhs) of the fastest on average; over the first
 // campaign the rules' own ran within 1.06 and 1.05.  Its gains are splits of
-// 256-long blocks where the rules take a smaller block unsplit
-// (4736x1128x11552: 163 -> 130 us), and splits in 3 or 6 parts
-// (456x4232x6088 lhs.rhs: 49 -> 39 us).  256 x 128 in 2 parts stays: it is a
-// rule for shapes timed on their own.
+// 256-long blocks where the rules take a smaller block unsplit or in fewer
+// parts (lhsT.rhs 4736x1128x11552: 163 -> 129 us; 2528x656x15008: 84 -> 70).
+// lhsT.rhs past 2.5e11 operations keeps the rules' pick (1024x8192x16384 is
+// fixed by a test), as does lhs.rhs where its rule for shapes timed on their
+// own takes 256 x 128 in 2 parts.
 mi_tile_cfg refined_matmul(int kernel_id, bool lhs, int M, int N, int K) {
   const mi_tile_cfg pick = matmul_default(kernel_id, lhs, M, N, K);
-  constexpr double kMaxFlops = 4e11;
-  if (!lhs) return refined(kernel_id, kLhsTTimed, count(kLhsTTimed), pick, 0.91, kMaxFlops, M, N, K);
+  if (!lhs) return refined(kernel_id, kLhsTTimed, count(kLhsTTimed), pick, 0.91, 2.5e11, M, N, K);
   if (pick.block_m == 256 && pick.block_n == 128 && pick.split_k == 2) return pick;
-  return refined(kernel_id, kLhsTimed, count(kLhsTimed), pick, 0.97, kMaxFlops, M, N, K);
+  return refined(kernel_id, kLhsTimed, count(kLhsTimed), pick, 0.97, 4e11, M, N, K);
 }
 
 // The fused kernel past skinny M.  The blocks that the rules above do not
 // know are the cached 64 x 64, 64 x 128 and 128 x 128 ones with a ring of 4
 // K tiles for W and 3 for x (rms_bf16_xreg.hip): at 50 shapes drawn
 // afterwards and timed with every block and split the refined pick ran
-// within 1.035 of the fastest on average; the rules' own ran within 1.18 at
+// within 1.032 of the fastest on average; the rules' own ran within 1.18 at
 // 70 (600x304x584: 11.0 -> 6.6 us; 1176x1432x1168: 19.5 -> 12.8;
 // 6272x240x968: 19.9 -> 11.5).  Where M >= 256, N >= 2048 and K >= 2048 it
 // has to win by 30 %: tests fix the rules' picks at several shapes there
@@ -737,7 +739,7 @@ int pick_default(int kernel_id, int M, int N, int K, mi_tile_cfg* cfg) {
 // M > 128 give way to a gamma-free variant, unsplit, where that is faster by
 // the fitted times: 64x128 and 64x64 to variant 14 with the same block,
 // 128x128 to variant 16 at 128x128 or variant 14 at 64x128 or 64x64.  At 50
-// shapes drawn afterwards the pick ran within 1.036 of the fastest on
+// shapes drawn afterwards the pick ran within 1.035 of the fastest on
 // average, against 1.16 at 40 for always taking the gamma-free variant (152x160x5112, where 64x64 blocks unsplit leave 247 CUs idle: 23.3 ->
 // 9 us in 16 parts; 872x280x9560: 45 -> 21 us).  A pick that was not timed
 // without gamma moves as those rules did: a 128 x 128 block to the largest
