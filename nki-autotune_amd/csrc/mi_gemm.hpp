@@ -581,32 +581,41 @@ struct PipeCfg {
 // Split-K epilogue: part p stores its fp32 accumulators to ws[p][M][N].
 // Lane l holds row l%32 of each 32x32 fragment, four consecutive columns per
 // dword quad, so a store from registers would touch 32 rows of 32 bytes;
-// each wave turns its fragments in its own piece of LDS instead (32 rows,
+// each wave turns its fragments in its own piece of LDS instead (ROWS rows,
 // stride 144 bytes; wave-private, so no barrier) and stores 8 rows of whole
-// 128-byte lines.  N % 8 == 0, so a quad is in bounds whenever its first
+// 128-byte lines.  ROWS is 32, or 16 where the panel buffers are too small
+// for 32 (64 x 64 blocks of 4 waves with two stages of block_k 32; the bf16
+// epilogue's own 2560 bytes per wave always hold 16).  N % 8 == 0, so a quad is in bounds whenever its first
 // column is.  A second kernel sums the parts.
-constexpr int kPartialRow = 144, kPartialSlot = 32 * kPartialRow;
-template <int TM, int TN>
+constexpr int kPartialRow = 144;
+constexpr int partial_rows(int waves, int lds_bytes) { return waves * 32 * kPartialRow <= lds_bytes ? 32 : 16; }
+template <int TM, int TN, int ROWS>
 __device__ __forceinline__ void store_partial(const f32x16_t (&acc)[TM][TN], float* __restrict__ ws, char* smem,
                                               int wave, int lane, int M, int N, int row0, int col0) {
-  MI_LDS char* slot = (MI_LDS char*)smem + wave * kPartialSlot;
+  MI_LDS char* slot = (MI_LDS char*)smem + wave * (ROWS * kPartialRow);
+  const int row = lane & 31;
 #pragma unroll
   for (int mt = 0; mt < TM; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < TN; ++nt) {
+    for (int nt = 0; nt < TN; ++nt)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const f32x4_t v = {acc[mt][nt][4 * j], acc[mt][nt][4 * j + 1], acc[mt][nt][4 * j + 2], acc[mt][nt][4 * j + 3]};
-        *(MI_LDS f32x4_t*)(slot + (lane & 31) * kPartialRow + 32 * j + 16 * (lane >> 5)) = v;
-      }
-      const int n = col0 + nt * 32 + 4 * (lane & 7);
+      for (int h = 0; h < 32 / ROWS; ++h) {
+        if (ROWS == 32 || row / ROWS == h) {
 #pragma unroll
-      for (int it = 0; it < 4; ++it) {
-        const int r = it * 8 + (lane >> 3), m = row0 + mt * 32 + r;
-        const f32x4_t v = *(MI_LDS f32x4_t*)(slot + r * kPartialRow + 16 * (lane & 7));
-        if (m < M && n < N) *(f32x4_t*)(ws + (size_t)m * N + n) = v;
+          for (int j = 0; j < 4; ++j) {
+            const f32x4_t v = {acc[mt][nt][4 * j], acc[mt][nt][4 * j + 1], acc[mt][nt][4 * j + 2],
+                               acc[mt][nt][4 * j + 3]};
+            *(MI_LDS f32x4_t*)(slot + row % ROWS * kPartialRow + 32 * j + 16 * (lane >> 5)) = v;
+          }
+        }
+        const int n = col0 + nt * 32 + 4 * (lane & 7);
+#pragma unroll
+        for (int it = 0; it < ROWS / 8; ++it) {
+          const int r = it * 8 + (lane >> 3), m = row0 + mt * 32 + h * ROWS + r;
+          const f32x4_t v = *(MI_LDS f32x4_t*)(slot + r * kPartialRow + 16 * (lane & 7));
+          if (m < M && n < N) *(f32x4_t*)(ws + (size_t)m * N + n) = v;
+        }
       }
-    }
 }
 
 // Epilogue of the K-split-over-waves core: every wave holds the whole
@@ -1050,8 +1059,10 @@ __device__ __forceinline__ void mm_pipe_body(const uint16_t* __restrict__ a, con
     return;
   }
   if constexpr (SPLIT) {
-    static_assert(WAVES * kPartialSlot <= C::LDS_BYTES, "the waves' pieces fit the panel buffers");
-    store_partial<TM, TN>(acc, sk.ws + (size_t)part * (size_t)M * (size_t)N, smem, wave, lane, M, N, m0 + wm0, n0 + wn0);
+    constexpr int ROWS = partial_rows(WAVES, C::LDS_BYTES);
+    static_assert(WAVES * ROWS * kPartialRow <= C::LDS_BYTES, "the waves' pieces fit the panel buffers");
+    store_partial<TM, TN, ROWS>(acc, sk.ws + (size_t)part * (size_t)M * (size_t)N, smem, wave, lane, M, N, m0 + wm0,
+                                n0 + wn0);
     return;
   }
   if constexpr (SK) {

@@ -378,8 +378,9 @@ __global__ __launch_bounds__(WAVES * 64) void rmsnorm_mm_bf16_xreg_kernel(
       const int m = m0 + xrow[i];
       if (tni == 0 && kc == 0 && m < M) ws[(size_t)parts * M * N + (size_t)part * M + m] = r;
     }
-    static_assert(WAVES * kPartialSlot <= C::MAIN_BYTES, "the waves' pieces fit the panel buffers");
-    store_partial<TM, TN>(acc, ws + (size_t)part * M * N, smem, wave, lane, M, N, m0 + wm0, n0 + wn0);
+    constexpr int ROWS = partial_rows(WAVES, C::RMS_OFF);
+    static_assert(WAVES * ROWS * kPartialRow <= C::RMS_OFF, "the waves' pieces fit the panel buffers");
+    store_partial<TM, TN, ROWS>(acc, ws + (size_t)part * M * N, smem, wave, lane, M, N, m0 + wm0, n0 + wn0);
     return;
   }
 #pragma unroll
