@@ -58,7 +58,9 @@ enum {
  * knobs (tbm/tbn/tbk, dim_order, multi-buffer counts;
  * reference kernel_library/README.md:12-13,
  * kernel_library/matmul/lhsT_rhs/kernel_hand_90.92mfu.py:107-112).
- *   block_m, block_n, block_k : workgroup tile (output rows, cols, K panel)
+ *   block_m, block_n, block_k : workgroup tile (output rows, cols, K panel):
+ *                               powers of two; rows and cols also 192 in
+ *                               variant 1 of the bf16 products
  *   waves                     : wavefronts (64 lanes) per workgroup
  *   lds_stages                : LDS ring depth for K panels (1..4); for matmul
  *                               variant 2 the depth of its register ring

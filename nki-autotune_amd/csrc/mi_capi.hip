@@ -137,26 +137,31 @@ using mi::capi::splittable;
 // predicates the kernel templates assert when they are instantiated).
 mi::Legal template_legal(int kernel_id, const mi_tile_cfg& c) {
   const int bm = c.block_m, bn = c.block_n, bk = c.block_k, w = c.waves, s = c.lds_stages;
+  // Blocks 192 wide are built for the cached products (variant 1 of each) only.
+  const auto pow2_only = [&](const mi::Legal& l) {
+    return bm == 192 || bn == 192 ? mi::bad(MI_E_TILE, "this variant takes blocks of powers of two in [32, 512]") : l;
+  };
   switch (kernel_id) {
     case MI_KERNEL_MATMUL_LHST_RHS_BF16:
       if (c.variant == 0) return mi::legal_mm_plain(bm, bn, bk, w, s);
-      if (c.variant == 1 || c.variant == 3) return mi::legal_mm_pipe(bm, bn, bk, w, s, false);
+      if (c.variant == 1) return mi::legal_mm_pipe(bm, bn, bk, w, s, false);
+      if (c.variant == 3) return pow2_only(mi::legal_mm_pipe(bm, bn, bk, w, s, false));
       if (c.variant == 2) return mi::legal_mm_reg(bm, bn, bk, w, s);
       if (c.variant == 4) return mi::legal_mm_kw(bm, bn, bk, w, s);
-      if (c.variant == 5 || c.variant == 6) return mi::legal_mm_pipe(bm, bn, bk, w, s, false);
+      if (c.variant == 5 || c.variant == 6) return pow2_only(mi::legal_mm_pipe(bm, bn, bk, w, s, false));
       break;
     case MI_KERNEL_MATMUL_LHS_RHS_BF16:
-      if (c.variant == 0 || c.variant == 2) return mi::legal_mm_pipe(bm, bn, bk, w, s, true);
+      if (c.variant == 0 || c.variant == 2) return pow2_only(mi::legal_mm_pipe(bm, bn, bk, w, s, true));
       if (c.variant == 1) return mi::legal_lhs_pair(bm, bn, bk, w, s);
       break;
     case MI_KERNEL_RMSNORM_MATMUL_BF16:
       if (c.variant == 0 || c.variant == 1) return mi::legal_rms_plain(bm, bn, bk, w, s);
       if (c.variant == 4 || c.variant == 5) return mi::legal_rms_xreg(bm, bn, bk, w, s, c.variant - 2);
       if (c.variant == 11 || c.variant == 12) return mi::legal_rms_xreg(bm, bn, bk, w, s, c.variant - 9);
-      if (c.variant == 13) return mi::legal_rms2(bm, bn, bk, w, s);
-      if (c.variant == 15) return mi::legal_rms2_pair(bm, bn, bk, w, s);
-      if (c.variant == 14) return mi::legal_mm_pipe(bm, bn, bk, w, s, true);
-      if (c.variant == 16) return mi::legal_lhs_pair(bm, bn, bk, w, s);
+      if (c.variant == 13) return pow2_only(mi::legal_rms2(bm, bn, bk, w, s));
+      if (c.variant == 15) return pow2_only(mi::legal_rms2_pair(bm, bn, bk, w, s));
+      if (c.variant == 14) return pow2_only(mi::legal_mm_pipe(bm, bn, bk, w, s, true));
+      if (c.variant == 16) return pow2_only(mi::legal_lhs_pair(bm, bn, bk, w, s));
       break;
     case MI_KERNEL_MATMUL_LHST_RHS_F32:
       // 16 x 16 threads with 4 x 4 outputs each, K slices of 16 or 32.

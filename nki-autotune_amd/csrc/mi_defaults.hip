@@ -498,6 +498,21 @@ const Timed kLhsTimed[] = {
     {{128, 128, 32, 4, 4, 1, 8, 1}, 2.08, 1.41, 0.168, 0.955, 0.444, 0.407, 0.0282, 0, 0, 0, 0},
 };
 
+// Blocks 192 wide, fitted the same way at 120 lhsT.rhs and 140 lhs.rhs shapes
+// with M > 128 and up to 4e11 operations.
+const Timed kLhsT192Timed[] = {
+    {{192, 256, 32, 4, 3, 1, 8, 1}, 0.783, 6.26, 0.277, 1.09, 0.748, 0.449, 0.0747, 2.43, 0.681, 0, 0},
+    {{192, 192, 32, 4, 3, 1, 8, 1}, 1.25, 4.7, 0.194, 0.978, 0.723, 1.41, 0.0803, 2.54, 0.9, 0, 0},
+    {{192, 128, 32, 4, 3, 1, 8, 1}, 1.42, 2.88, 0.187, 0.968, 0.486, 0.787, 0.0707, 2.64, 0.91, 0, 0},
+    {{128, 192, 32, 4, 3, 1, 8, 1}, 1.2, 3.11, 0.183, 0.899, 0.635, 0.534, 0.0538, 2.67, 1.02, 0, 0},
+};
+const Timed kLhs192Timed[] = {
+    {{192, 256, 32, 8, 3, 1, 8, 1}, 0.295, 5.7, 0.253, 1.11, 0.873, 0.162, 0.109, 0, 0, 0, 0},
+    {{192, 192, 32, 4, 3, 1, 8, 1}, 1.01, 4.54, 0.273, 1.09, 0.589, 0.146, 0.0776, 0, 0, 0, 0},
+    {{192, 128, 32, 4, 4, 1, 8, 1}, 0.718, 3.34, 0.225, 1.03, 0.462, 0.284, 0.117, 0, 0, 0, 0},
+    {{128, 192, 32, 4, 4, 1, 8, 1}, 0.811, 3.41, 0.211, 1.06, 0.554, 0.406, 0.0571, 0, 0, 0, 0},
+};
+
 // M <= 128 with a weight of at most 7 MiB, and (lhs.rhs, non-temporal blocks
 // only) of 7 to 28 MiB: the same fits to 160 shapes of each kind (120 for
 // the last), the weight warm in the caches as a call repeated over a few
@@ -583,15 +598,11 @@ bool runs_split(int kernel_id, const mi_tile_cfg& c, int parts, int M, int N, in
   return mi::workspace_bytes(kernel_id, p, M, N, K, kDefaultCus) <= kMaxWorkspace;
 }
 
-// `pick` (what the rules above choose), or the candidate of `table` with the
-// least fitted time where that is under `margin` of the pick's own fitted
-// time.  A pick that was not timed stays, and so does every pick of a call
-// past the timed range.
-mi_tile_cfg refined(int kernel_id, const Timed* table, int n, const mi_tile_cfg& pick, double margin, double max_flops,
-                    int M, int N, int K) {
-  const Timed* old = timed(table, n, pick);
-  if (!old || 2.0 * M * N * K > max_flops) return pick;
-  double best_t = margin * fitted_time(*old, pick.split_k, M, N, K);
+// `pick`, whose fitted coefficients are `old`, or the candidate of `table`
+// with the least fitted time where that is under `margin` of the pick's own.
+mi_tile_cfg faster_of(int kernel_id, const Timed* table, int n, const Timed& old, const mi_tile_cfg& pick, double margin,
+                      int M, int N, int K) {
+  double best_t = margin * fitted_time(old, pick.split_k, M, N, K);
   mi_tile_cfg best = pick;
   for (int i = 0; i < n; ++i) {
     for (const int parts : {1, 2, 3, 4, 5, 6, 7, 8, 12, 16}) {
@@ -604,6 +615,16 @@ mi_tile_cfg refined(int kernel_id, const Timed* table, int n, const mi_tile_cfg&
     }
   }
   return best;
+}
+
+// `pick` (what the rules above choose), or a candidate of `table` that
+// contains it (faster_of).  A pick that was not timed stays, and so does
+// every pick of a call past the timed range.
+mi_tile_cfg refined(int kernel_id, const Timed* table, int n, const mi_tile_cfg& pick, double margin, double max_flops,
+                    int M, int N, int K) {
+  const Timed* old = timed(table, n, pick);
+  if (!old || 2.0 * M * N * K > max_flops) return pick;
+  return faster_of(kernel_id, table, n, *old, pick, margin, M, N, K);
 }
 
 // fp32: the MFMA kernel with K split over the waves (variant 3; variants 0,
@@ -687,11 +708,32 @@ mi_tile_cfg refined_skinny(int kernel_id, int M, int N, int K) {
 // lhsT.rhs past 2.5e11 operations keeps the rules' pick (1024x8192x16384 is
 // fixed by a test), as does lhs.rhs where its rule for shapes timed on their
 // own takes 256 x 128 in 2 parts.
+//
+// Blocks 192 wide come last: they win where the other blocks leave CUs idle
+// in the last round (lhs.rhs 1000x5000x4104: 160 tiles of 128 x 256 leave 96
+// idle, 216 of 128 x 192 leave 40, 50.7 -> 46.5 us; lhsT.rhs 2056x4032x8520:
+// 144 tiles of 256 x 256 against 231 of 192 x 192, 161 -> 133 us).  They
+// change 10 of 120 picks timed (lhsT.rhs, 1.21 x faster on average, 1.07 at
+// least) and 12 of 140 (lhs.rhs, 1.14 and 1.08), and at 16 changed picks of
+// each drawn afterwards 1.11 (1.04 at least) and 1.12 x (1.04).  Below
+// K = 512 the fits miss by up to 20 % and the picks stay; so do lhsT.rhs
+// picks already split (which fill the chip: 1.10 x at one of 120 shapes) and
+// 256 x 256 and 64 x 256 blocks without padded rows: tests fix those at
+// 3072^3, where 256 tiles of 192 x 192 would fill the one round that 144 of
+// 256 x 256 do not, and at 1088x3712x8000.
 mi_tile_cfg refined_matmul(int kernel_id, bool lhs, int M, int N, int K) {
-  const mi_tile_cfg pick = matmul_default(kernel_id, lhs, M, N, K);
-  if (!lhs) return refined(kernel_id, kLhsTTimed, count(kLhsTTimed), pick, 0.91, 2.5e11, M, N, K);
-  if (pick.block_m == 256 && pick.block_n == 128 && pick.split_k == 2) return pick;
-  return refined(kernel_id, kLhsTimed, count(kLhsTimed), pick, 0.97, 4e11, M, N, K);
+  const mi_tile_cfg rules = matmul_default(kernel_id, lhs, M, N, K);
+  if (lhs && rules.block_m == 256 && rules.block_n == 128 && rules.split_k == 2) return rules;
+  constexpr double kMaxFlops = 4e11;
+  const Timed* table = lhs ? kLhsTimed : kLhsTTimed;
+  const int n = lhs ? count(kLhsTimed) : count(kLhsTTimed);
+  const mi_tile_cfg pick = refined(kernel_id, table, n, rules, lhs ? 0.97 : 0.91, lhs ? kMaxFlops : 2.5e11, M, N, K);
+  const Timed* old = timed(table, n, pick);
+  if (!old || K < 512 || 2.0 * M * N * K > kMaxFlops) return pick;
+  if (lhs) return faster_of(kernel_id, kLhs192Timed, count(kLhs192Timed), *old, pick, 0.97, M, N, K);
+  const bool fixed = pick.block_n == 256 && pick.block_m != 128 && M % pick.block_m == 0;
+  if (pick.split_k > 1 || fixed) return pick;
+  return faster_of(kernel_id, kLhsT192Timed, count(kLhsT192Timed), *old, pick, 0.95, M, N, K);
 }
 
 // The fused kernel past skinny M.  The blocks that the rules above do not

@@ -213,19 +213,26 @@ __device__ __forceinline__ int mn_swz(int k) {
   else return half & (ROWB / 16 - 1);
 }
 
+// Columns of one LDS panel of a block W wide: all of them where W is a power
+// of two; a width of 192 is laid out as three panels of 64 (128-byte rows,
+// one after the other), each swizzled by itself.
+constexpr int panel_cols(int w) { return (w & (w - 1)) == 0 ? w : 64; }
+
 // LDS-direct loader of one [BK][W] MN-contiguous panel (W = BM or BN):
 // the panel is CH = BK*W*2/1024 chunks of 1 KiB; one wave instruction fills
 // one chunk, lane l writing bytes [16l, 16l+16).  The lane fetches the
 // global 16 bytes that the swizzle maps to that LDS position.
 template <int BK, int W, int WAVES>
 struct PanelLoader {
-  static constexpr int ROWB = W * 2;
+  static constexpr int PW = panel_cols(W);
+  static constexpr int ROWB = PW * 2;
   static constexpr int CH = BK * W * 2 / 1024;
+  static constexpr int CH_PER_PANEL = BK * ROWB / 1024;
   static constexpr int PER_WAVE = (CH + WAVES - 1) / WAVES;
-  static constexpr int LANES_PER_ROW = W / 8;  // 16-byte slots per K row
+  static constexpr int LANES_PER_ROW = PW / 8;  // 16-byte slots per K row
   static constexpr int ROWS_PER_CH = 1024 / ROWB;
   static constexpr bool EVEN = CH % WAVES == 0;  // every wave issues PER_WAVE loads
-  static_assert(W >= 32 && (W & (W - 1)) == 0, "panel width must be a power of two >= 32");
+  static_assert(W >= 32 && W % PW == 0 && CH_PER_PANEL >= 1, "panels of a power of two >= 32 columns");
   static_assert(CH >= 1, "panel smaller than one wave load");
   static_assert(ROWB <= 1024, "panel row wider than one wave load");
   uint32_t voff[PER_WAVE];  // per-lane byte offset at K tile 0
@@ -237,10 +244,11 @@ struct PanelLoader {
     for (int j = 0; j < PER_WAVE; ++j) {
       const int c = wave + j * WAVES;
       active[j] = c < CH;
-      const int row = c * ROWS_PER_CH + lane / LANES_PER_ROW;
+      const int panel = PW == W ? 0 : c / CH_PER_PANEL;
+      const int row = (c - panel * CH_PER_PANEL) * ROWS_PER_CH + lane / LANES_PER_ROW;
       const int slot = lane % LANES_PER_ROW;
       const int q = slot ^ mn_swz<ROWB>(row);
-      voff[j] = ((uint32_t)row * (uint32_t)ld + (uint32_t)(col0 + 8 * q)) * 2u;
+      voff[j] = ((uint32_t)row * (uint32_t)ld + (uint32_t)(col0 + panel * PW + 8 * q)) * 2u;
       lds_off[j] = c * 1024;
     }
   }
@@ -330,17 +338,21 @@ struct KPanelLoader {
 // ds_read_b64_tr_b16 from an MN-contiguous [BK][W] panel.  For fragment t
 // (32 columns starting at w0 + 32t) and K sub-step kk, half h, the address
 // is panel + (kk*16 + 4h) * ROWB + off[t].
-template <int W, int T>
+// BK: rows of the panel, needed where W takes more than one.
+template <int W, int T, int BK = 0>
 struct TrFrag {
-  static constexpr int ROWB = W * 2;
+  static constexpr int PW = panel_cols(W);
+  static constexpr int ROWB = PW * 2;
+  static_assert(PW == W || BK > 0, "the panels' stride");
   int off[T];
   __device__ __forceinline__ void init(int lane, int w0) {
     const int g = lane >> 4, i = lane & 15, r = i >> 2, c = i & 3;
     const int krow = 8 * (g >> 1) + r;  // K row inside the 16-row sub-step
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-      const int col = w0 + 32 * t + 16 * (g & 1) + 4 * c;
-      off[t] = krow * ROWB + 16 * ((col >> 3) ^ mn_swz<ROWB>(krow)) + (col & 7) * 2;
+      const int wcol = w0 + 32 * t + 16 * (g & 1) + 4 * c;
+      const int panel = PW == W ? 0 : wcol / PW, col = wcol - panel * PW;
+      off[t] = panel * (BK * ROWB) + krow * ROWB + 16 * ((col >> 3) ^ mn_swz<ROWB>(krow)) + (col & 7) * 2;
     }
   }
 };
@@ -371,7 +383,7 @@ __device__ __forceinline__ void store_tile(f32x16_t (&acc)[TM][TN], const float 
   constexpr int WTN = TN * 32;
   constexpr int SROW = WTN * 2 + 16;
   constexpr int CPR = WTN / 8;       // 16-byte chunks per row
-  constexpr int RPI = 64 / CPR;      // rows per read instruction
+  static_assert(32 * CPR % 64 == 0, "whole read instructions per slice");
   char* ep = smem + wave * (32 * SROW);
 #pragma unroll
   for (int mt = 0; mt < TM; ++mt) {
@@ -390,9 +402,9 @@ __device__ __forceinline__ void store_tile(f32x16_t (&acc)[TM][TN], const float 
     }
     __syncthreads();
 #pragma unroll
-    for (int it = 0; it < 32 / RPI; ++it) {
-      const int rl = it * RPI + lane / CPR;
-      const int cl = lane % CPR;
+    for (int it = 0; it < 32 * CPR / 64; ++it) {
+      const int rl = (it * 64 + lane) / CPR;
+      const int cl = (it * 64 + lane) % CPR;
       const u32x4_t v = *(MI_LDS u32x4_t*)((MI_LDS char*)ep + rl * SROW + cl * 16);
       const int m = row0 + mt * 32 + rl;
       const int n = col0 + cl * 8;
@@ -818,8 +830,10 @@ __device__ __forceinline__ void mm_pipe_body(const uint16_t* __restrict__ a, con
   lb.init(wave, lane, n0, N);
   const uint32_t kstep_a = AK ? (uint32_t)BK * 2u : (uint32_t)BK * (uint32_t)M * 2u;
   const uint32_t kstep_b = (uint32_t)BK * (uint32_t)N * 2u;
-  TrFrag<BM, TM> fa;
-  TrFrag<BN, TN> fb;
+  using FA = TrFrag<BM, TM, BK>;
+  using FB = TrFrag<BN, TN, BK>;
+  FA fa;
+  FB fb;
   if constexpr (!AK) fa.init(lane, wm0);
   fb.init(lane, wn0);
   if constexpr (KW) {
@@ -827,9 +841,9 @@ __device__ __forceinline__ void mm_pipe_body(const uint16_t* __restrict__ a, con
     // operand swizzle repeats every 16 rows, so a row offset is enough).
     const int kb = wave * KSW * 16;
 #pragma unroll
-    for (int t = 0; t < TM; ++t) fa.off[t] += kb * (BM * 2);
+    for (int t = 0; t < TM; ++t) fa.off[t] += kb * FA::ROWB;
 #pragma unroll
-    for (int t = 0; t < TN; ++t) fb.off[t] += kb * (BN * 2);
+    for (int t = 0; t < TN; ++t) fb.off[t] += kb * FB::ROWB;
   }
   // K-contiguous A operand: lane l reads row l%32 of the fragment, K chunk
   // 2*kk + l/32 of the sub-step, at its k_swz slot (the same for every
@@ -858,12 +872,12 @@ __device__ __forceinline__ void mm_pipe_body(const uint16_t* __restrict__ a, con
         af[buf][t] = __builtin_bit_cast(
             bf16x8_t, *(MI_LDS u32x4_t*)((MI_LDS char*)smem + abase + arow + t * 32 * (BK * 2) + akoff[kk]));
       else
-        af[buf][t] = read_tr_frag(smem, abase + (kk * 16) * (BM * 2) + fa.off[t],
-                                  abase + (kk * 16 + 4) * (BM * 2) + fa.off[t]);
+        af[buf][t] = read_tr_frag(smem, abase + (kk * 16) * FA::ROWB + fa.off[t],
+                                  abase + (kk * 16 + 4) * FA::ROWB + fa.off[t]);
     } else {
       const int t = f - 1;
-      bf[buf][t] = read_tr_frag(smem, bbase + (kk * 16) * (BN * 2) + fb.off[t],
-                                bbase + (kk * 16 + 4) * (BN * 2) + fb.off[t]);
+      bf[buf][t] = read_tr_frag(smem, bbase + (kk * 16) * FB::ROWB + fb.off[t],
+                                bbase + (kk * 16 + 4) * FB::ROWB + fb.off[t]);
     }
   };
   auto read_frags = [&](int stage, int kk, int buf) {

@@ -60,7 +60,9 @@ MI_HD constexpr int epilogue_bytes(int bm, int bn, int waves) {
 // LDS-direct loader of an MN-contiguous [bk][w] panel (PanelLoader): rows of
 // at most 1 KiB, at least one 1 KiB chunk; `even` when every wave issues the
 // same number of chunk loads.
-MI_HD constexpr bool mn_panel_ok(int bk, int w) { return w >= 32 && is_pow2(w) && w * 2 <= 1024 && bk * w * 2 >= 1024; }
+MI_HD constexpr bool mn_panel_ok(int bk, int w) {
+  return ((w >= 32 && is_pow2(w)) || w == 192) && w * 2 <= 1024 && bk * w * 2 >= 1024;
+}
 MI_HD constexpr int mn_panel_loads(int bk, int w, int waves) { return (bk * w * 2 / 1024 + waves - 1) / waves; }
 MI_HD constexpr bool mn_panel_even(int bk, int w, int waves) { return (bk * w * 2 / 1024) % waves == 0; }
 
@@ -74,6 +76,11 @@ MI_HD constexpr bool k_panel_even(int bk, int rows, int waves) { return (rows * 
 // Block sizes every bf16 template takes: powers of two, 32..512 wide.
 MI_HD constexpr bool block_mn_ok(int bm, int bn) {
   return is_pow2(bm) && is_pow2(bn) && bm >= 32 && bm <= 512 && bn >= 32 && bn <= 512;
+}
+// The pipelined and paired-load cores also take blocks 192 wide (three
+// panels of 64).
+MI_HD constexpr bool block_mn_or_192_ok(int bm, int bn) {
+  return block_mn_ok(bm == 192 ? 64 : bm, bn == 192 ? 64 : bn);
 }
 MI_HD constexpr bool waves_ok(int waves) { return is_pow2(waves) && waves <= 16; }
 
@@ -112,8 +119,8 @@ MI_HD constexpr int lds_mm_pipe(int bm, int bn, int bk, int waves, int stages) {
   return cmax(stages * (bk * bm * 2 + bk * bn * 2), epilogue_bytes(bm, bn, waves));
 }
 MI_HD constexpr Legal legal_mm_pipe(int bm, int bn, int bk, int waves, int stages, bool ak) {
-  if (!block_mn_ok(bm, bn) || !is_pow2(bk) || bk < 32 || bk > 128)
-    return bad(MI_E_TILE, "block_m, block_n must be powers of two in [32, 512] and block_k in [32, 128]");
+  if (!block_mn_or_192_ok(bm, bn) || !is_pow2(bk) || bk < 32 || bk > 128)
+    return bad(MI_E_TILE, "block_m, block_n must be powers of two in [32, 512] or 192, and block_k in [32, 128]");
   if (wave_rules(bm, bn, waves).code != MI_OK) return wave_rules(bm, bn, waves);
   if (stages < 2 || stages > 4) return bad(MI_E_TILE, "this variant takes 2..4 LDS stages");
   const bool a_ok = ak ? k_panel_ok(bk, bm) : mn_panel_ok(bk, bm);
@@ -211,8 +218,8 @@ MI_HD constexpr int lds_lhs_pair(int bm, int bn, int bk, int waves, int stages) 
   return cmax(((stages + 2) / 2) * (bm * 2 * bk * 2) + stages * (bk * bn * 2), epilogue_bytes(bm, bn, waves));
 }
 MI_HD constexpr Legal legal_lhs_pair(int bm, int bn, int bk, int waves, int stages) {
-  if (!block_mn_ok(bm, bn) || (bk != 32 && bk != 64))
-    return bad(MI_E_TILE, "block_m, block_n must be powers of two in [32, 512] and block_k 32 or 64");
+  if (!block_mn_or_192_ok(bm, bn) || (bk != 32 && bk != 64))
+    return bad(MI_E_TILE, "block_m, block_n must be powers of two in [32, 512] or 192, and block_k 32 or 64");
   if (wave_rules(bm, bn, waves).code != MI_OK) return wave_rules(bm, bn, waves);
   if (stages < 2 || stages > 4) return bad(MI_E_TILE, "this variant takes 2..4 LDS stages");
   if (!k_panel_ok(2 * bk, bm) || !mn_panel_ok(bk, bn)) return bad(MI_E_TILE, "a K panel is smaller than one 1 KiB wave load");

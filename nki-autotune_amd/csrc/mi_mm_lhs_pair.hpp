@@ -110,7 +110,8 @@ __device__ __forceinline__ void mm_lhs_pair_body(const uint16_t* __restrict__ lh
   lb.init(wave, lane, n0, N);
   const uint32_t kstep_pair = (uint32_t)(2 * BK) * 2u;
   const uint32_t kstep_b = (uint32_t)BK * (uint32_t)N * 2u;
-  TrFrag<BN, TN> fb;
+  using FB = TrFrag<BN, TN, BK>;
+  FB fb;
   fb.init(lane, wn0);
   // A operand: lane l reads row l%32 of a fragment, K chunk h*KC + 2*kk +
   // l/32 of the pair row (h: which tile of the pair), at its k_swz slot.
@@ -140,8 +141,8 @@ __device__ __forceinline__ void mm_lhs_pair_body(const uint16_t* __restrict__ lh
     } else {
       const int t = f - 1;
       const int bbase = C::B_OFF + stage * C::B_BYTES;
-      bf[buf][t] = read_tr_frag(smem, bbase + (kk * 16) * (BN * 2) + fb.off[t],
-                                bbase + (kk * 16 + 4) * (BN * 2) + fb.off[t]);
+      bf[buf][t] = read_tr_frag(smem, bbase + (kk * 16) * FB::ROWB + fb.off[t],
+                                bbase + (kk * 16 + 4) * FB::ROWB + fb.off[t]);
     }
   };
   auto read_frags = [&](int stage, int pb, int h, int kk, int buf) {

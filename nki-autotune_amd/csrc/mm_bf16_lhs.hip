@@ -44,7 +44,11 @@
   X(128, 256, 32, 4, 3)        \
   X(128, 256, 64, 4, 2)        \
   X(128, 128, 64, 4, 3)        \
-  X(128, 128, 32, 4, 4)
+  X(128, 128, 32, 4, 4)        \
+  X(192, 256, 32, 8, 3)        \
+  X(192, 192, 32, 4, 3)        \
+  X(128, 192, 32, 4, 4)        \
+  X(192, 128, 32, 4, 4)
 
 #define MI_LHS_SKINNY_CONFIGS(X) \
   X(32, 128, 64, 4, 4)           \

@@ -37,12 +37,21 @@
   X(64, 64, 64, 4, 4)        \
   X(64, 128, 128, 4, 3)
 
+// Blocks 192 long (variant 1): outputs whose grid of 128- and 256-long
+// blocks leaves a round of the CUs nearly empty.
+#define MI_PIPE_192_CONFIGS(X) \
+  X(192, 256, 32, 4, 3)        \
+  X(192, 192, 32, 4, 3)        \
+  X(192, 128, 32, 4, 3)        \
+  X(128, 192, 32, 4, 3)
+
 namespace mi {
 MI_PIPE_CONFIGS(MI_MMP_INST)
 MI_PIPE_CONFIGS(MI_MMPN_INST)
+MI_PIPE_192_CONFIGS(MI_MMP_INST)
 
 const MiEntry* table_mm_pipe(int* n) {
-  static const MiEntry t[] = {MI_PIPE_CONFIGS(MI_MMP_ROW) MI_PIPE_CONFIGS(MI_MMPN_ROW)};
+  static const MiEntry t[] = {MI_PIPE_CONFIGS(MI_MMP_ROW) MI_PIPE_CONFIGS(MI_MMPN_ROW) MI_PIPE_192_CONFIGS(MI_MMP_ROW)};
   *n = (int)(sizeof(t) / sizeof(t[0]));
   return t;
 }
