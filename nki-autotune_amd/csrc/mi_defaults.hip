@@ -595,7 +595,10 @@ bool runs_split(int kernel_id, const mi_tile_cfg& c, int parts, int M, int N, in
   if (!e || (e->gamma_kmax > 0 && kts * c.block_k > e->gamma_kmax)) return false;
   mi_tile_cfg p = c;
   p.split_k = parts;
-  return mi::workspace_bytes(kernel_id, p, M, N, K, kDefaultCus) <= kMaxWorkspace;
+  // lhsT.rhs calls without a config also run from the no-allocation entry's
+  // static scratch, which 256 full blocks of 256 x 256 and the counters pass.
+  const unsigned long long cap = kernel_id == MI_KERNEL_MATMUL_LHST_RHS_BF16 ? MI_NOALLOC_SCRATCH_BYTES : kMaxWorkspace;
+  return mi::workspace_bytes(kernel_id, p, M, N, K, kDefaultCus) <= cap;
 }
 
 // `pick`, whose fitted coefficients are `old`, or the candidate of `table`
