@@ -158,17 +158,19 @@ int mi_get_config(int kernel_id, int idx, mi_tile_cfg* cfg);
  * variants for skinny M sized by an estimate of each workgroup's panel
  * bytes; for the fused kernel, the one-pass and two-pass kernels weighed by
  * the same estimate with their split and pack passes charged, past the K
- * its gamma staging holds split until each part's gamma fits.
+ * its gamma staging holds split until each part's gamma fits.  A block and
+ * split whose fitted time is enough under that pick's takes its place; fp32
+ * takes the block and wave count of the least estimated time.
  * A negative size is MI_E_ARGS. */
 int mi_default_config(int kernel_id, int M, int N, int K, mi_tile_cfg* cfg);
 
 /* The default of rmsnorm_matmul for a call without gamma (what
  * mi_rmsnorm_matmul_bf16 takes when cfg and gamma are both NULL):
- * mi_default_config's pick, except that its 64x128 and 64x64 blocks go to
- * the gamma-free variant 14 with the same block, and its 128x128 blocks to
- * the largest gamma-free block whose grid keeps more than half the CUs busy
- * (variant 16 at 128x128 with block_k 32 and 4 stages, else variant 14 at
- * 64x128, else at 64x64), all unsplit.
+ * mi_default_config's pick, except that at M > 128 its 128x128, 64x128 and
+ * 64x64 blocks give way to a gamma-free variant, unsplit, where that is
+ * faster by the fitted times: 64x128 and 64x64 to variant 14 with the same
+ * block, 128x128 to variant 16 (block_k 32, 4 stages) or to variant 14 at
+ * 64x128 or 64x64.
  * No counterpart in the reference, whose kernel has no gamma at all; for
  * callers of its contract (rmsnorm_matmul_online).  A negative size is
  * MI_E_ARGS. */
@@ -222,8 +224,8 @@ int mi_rmsnorm_matmul_bf16(const void* x, const void* gamma, const void* W, void
  * counters, then split_k * M * N * 4 bytes of fp32 partial products, or the
  * stream-K partial tiles) is a static device array of MI_NOALLOC_SCRATCH_BYTES
  * that each GPU holds from the first call there until the process ends, and
- * a config needing more returns MI_E_RANGE (cfg == NULL never does: the
- * default splits at most 256 blocks of 256 x 256).  Calls on one GPU share that
+ * a config needing more returns MI_E_RANGE (cfg == NULL never does: a
+ * default pick has to fit the scratch).  Calls on one GPU share that
  * array: calls ordered on one stream are safe, calls that overlap on one GPU
  * race. */
 #define MI_NOALLOC_SCRATCH_BYTES (64ull * 1024ull * 1024ull)
