@@ -586,19 +586,27 @@ struct PipeCfg {
   static constexpr int LDS_BYTES = MAIN_BYTES > EPI_BYTES ? MAIN_BYTES : EPI_BYTES;
 };
 
-// The pipelined body, for two layouts of the A operand: AK = false takes
-// lhsT[K,M] (M contiguous; MN-swizzled panel, transposing operand reads),
-// AK = true takes lhs[M,K] (K contiguous; K-swizzled panel, one
-// ds_read_b128 per operand fragment, no transpose).
+// Between LDS accesses of one wave where its lanes read what other lanes
+// wrote.  The LDS runs one wave's operations in order, but the compiler sees
+// only each thread's own addresses and may move an access over another
+// lane's; this keeps the two sides apart (no instruction, no workgroup
+// barrier).
+__device__ __forceinline__ void wave_lds_turn() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Split-K epilogue: part p stores its fp32 accumulators to ws[p][M][N].
 // Lane l holds row l%32 of each 32x32 fragment, four consecutive columns per
 // dword quad, so a store from registers would touch 32 rows of 32 bytes;
 // each wave turns its fragments in its own piece of LDS instead (ROWS rows,
-// stride 144 bytes; wave-private, so no barrier) and stores 8 rows of whole
+// stride 144 bytes; wave-private, so it takes no workgroup barrier, but a
+// wave_lds_turn on either side of the reads) and stores 8 rows of whole
 // 128-byte lines.  ROWS is 32, or 16 where the panel buffers are too small
 // for 32 (64 x 64 blocks of 4 waves with two stages of block_k 32; the bf16
-// epilogue's own 2560 bytes per wave always hold 16).  N % 8 == 0, so a quad is in bounds whenever its first
-// column is.  A second kernel sums the parts.
+// epilogue's own 2560 bytes per wave always hold 16).  N % 8 == 0, so a quad
+// is in bounds whenever its first column is.  A second kernel sums the parts.
 constexpr int kPartialRow = 144;
 constexpr int partial_rows(int waves, int lds_bytes) { return waves * 32 * kPartialRow <= lds_bytes ? 32 : 16; }
 template <int TM, int TN, int ROWS>
@@ -620,6 +628,7 @@ __device__ __forceinline__ void store_partial(const f32x16_t (&acc)[TM][TN], flo
             *(MI_LDS f32x4_t*)(slot + row % ROWS * kPartialRow + 32 * j + 16 * (lane >> 5)) = v;
           }
         }
+        wave_lds_turn();
         const int n = col0 + nt * 32 + 4 * (lane & 7);
 #pragma unroll
         for (int it = 0; it < ROWS / 8; ++it) {
@@ -627,6 +636,7 @@ __device__ __forceinline__ void store_partial(const f32x16_t (&acc)[TM][TN], flo
           const f32x4_t v = *(MI_LDS f32x4_t*)(slot + r * kPartialRow + 16 * (lane & 7));
           if (m < M && n < N) *(f32x4_t*)(ws + (size_t)m * N + n) = v;
         }
+        wave_lds_turn();
       }
 }
 
@@ -737,6 +747,10 @@ __global__ __launch_bounds__(256) void splitk_sum_kernel(const float* __restrict
 
 struct NoEpi {};
 
+// The pipelined body, for two layouts of the A operand: AK = false takes
+// lhsT[K,M] (M contiguous; MN-swizzled panel, transposing operand reads),
+// AK = true takes lhs[M,K] (K contiguous; K-swizzled panel, one
+// ds_read_b128 per operand fragment, no transpose).
 // SK (stream-K): the tile and its K range come from `seg`, and instead of an
 // epilogue of its own the body hands its accumulators to
 // epi(acc, row0, col0) (row0, col0: this wave's first output row and
