@@ -7,8 +7,10 @@ mdp.py:19-72) and samples it with a seeded, dedup'd frontier expansion
 a state is a :class:`~kernel_library.config.TileConfig` and an action (an
 "atom") changes one knob:
 
-* ``block_m`` / ``block_n`` / ``block_k`` doubled or halved,
-* ``waves`` 4 <-> 8,
+* ``block_m`` / ``block_n`` / ``block_k`` doubled or halved; the first two
+  also one width up or down where that leads to or from one that is no power
+  of two (128 - 192 - 256),
+* ``waves`` 4 <-> 8 (fp32: doubled or halved, 4 to 16),
 * ``lds_stages`` +1 / -1,
 * ``group_m`` (the L2 raster height) doubled or halved,
 * ``variant`` set to another pipeline of the same kernel family,
@@ -18,7 +20,12 @@ a state is a :class:`~kernel_library.config.TileConfig` and an action (an
 An atom is legal at a state when its result passes the library's static
 legality check at the problem shape (``mi_cfg_check``: LDS budget, wave
 tiling, alignment, 32-bit offsets, gamma capacity) and is either prebuilt
-or, unless ``prebuilt_only``, buildable from its variant's template.
+or, unless ``prebuilt_only``, buildable from its variant's template.  Where
+the variant has no such config with the other knobs unchanged (fp32's
+variants differ in stages, its 16-wide blocks in block_k, the 192-wide blocks
+of the two matmuls in stages), the move lands on the compiled config with the
+knob's new value that is nearest in the others, so every compiled config that
+is legal at the shape is reachable from every other.
 
 :func:`frontier_sample` keeps one pool of distinct configs (keyed by name)
 and a frontier of pool members with untried atoms; each step picks a
@@ -33,6 +40,7 @@ and the same seed gives the same configs.
 
 from __future__ import annotations
 
+import math
 import random
 from dataclasses import replace
 from typing import NamedTuple
@@ -44,7 +52,8 @@ from kernel_library.config import TileConfig
 
 
 class Atom(NamedTuple):
-    """One single-knob move: ``knob`` changed by ``op`` (``x2``, ``/2``, ``+1``, ``-1``, ``swap``, ``=<v>``)."""
+    """One single-knob move: ``knob`` changed by ``op`` (``x2``, ``/2``, ``+1``, ``-1``, ``swap``, ``wider``,
+    ``narrower``, ``=<v>``)."""
 
     knob: str
     op: str
@@ -59,15 +68,17 @@ FAMILY_VARIANTS = {
     "matmul_lhsT_rhs_f32": (0, 1, 3),
 }
 
-_POW2_KNOBS = {"block_m": (32, 512), "block_n": (32, 512), "block_k": (16, 128), "group_m": (1, 64),
-               "split_k": (1, 16)}
+_POW2_KNOBS = {"block_m": (16, 512), "block_n": (16, 512), "block_k": (16, 128), "group_m": (1, 64),
+               "split_k": (1, 16), "waves": (4, 16)}
 
 
 def atoms_for(func_name: str) -> list[Atom]:
     fam = canonical_name(func_name)
     out = [Atom(k, op) for k in ("block_m", "block_n", "block_k") for op in ("x2", "/2")]
-    out += [Atom("waves", "swap"), Atom("lds_stages", "+1"), Atom("lds_stages", "-1"),
-            Atom("group_m", "x2"), Atom("group_m", "/2")]
+    if fam in ("matmul_lhsT_rhs", "matmul_lhs_rhs"):
+        out += [Atom(k, op) for k in ("block_m", "block_n") for op in ("wider", "narrower")]
+    out += [Atom("waves", op) for op in (("x2", "/2") if fam == "matmul_lhsT_rhs_f32" else ("swap",))]
+    out += [Atom("lds_stages", "+1"), Atom("lds_stages", "-1"), Atom("group_m", "x2"), Atom("group_m", "/2")]
     out += [Atom("variant", f"={v}") for v in FAMILY_VARIANTS.get(fam, (0,))]
     if fam in ("matmul_lhsT_rhs", "matmul_lhs_rhs", "rmsnorm_matmul"):
         out += [Atom("split_k", "x2"), Atom("split_k", "/2")]
@@ -87,6 +98,7 @@ class TileMDP:
         self.prebuilt_only = prebuilt_only
         self.atoms = atoms_for(self.fam)
         self._legal: dict[str, bool] = {}
+        self._compiled = [c for c in kl.compiled_configs(self.fam) if c.variant in FAMILY_VARIANTS.get(self.fam, (0,))]
 
     def reset(self) -> TileConfig:
         """The library's default (tuned) config at the shape, with an explicit raster height."""
@@ -116,6 +128,10 @@ class TileMDP:
             nv = v - 1
         elif op == "swap":
             nv = 8 if v == 4 else 4
+        elif op in ("wider", "narrower"):
+            nv = {(128, "wider"): 192, (192, "wider"): 256, (256, "narrower"): 192, (192, "narrower"): 128}.get((v, op))
+            if nv is None:
+                raise IllegalMove(f"no width next to {v} that doubling or halving does not reach")
         elif op.startswith("="):
             nv = int(op[1:])
         else:
@@ -131,9 +147,30 @@ class TileMDP:
 
     def step(self, state: TileConfig, atom: Atom) -> TileConfig:
         nxt = self.apply(state, atom)
-        if not self.is_legal(nxt):
-            raise IllegalMove(f"{nxt.name} is illegal at {self.M}x{self.N}x{self.K}")
-        return nxt
+        if self.is_legal(nxt):
+            return nxt
+        if atom.knob not in ("group_m", "split_k"):
+            for cfg in self._nearest(state, nxt, atom.knob):
+                if cfg != state and self.is_legal(cfg):
+                    return cfg
+        raise IllegalMove(f"{nxt.name} is illegal at {self.M}x{self.N}x{self.K}")
+
+    def _nearest(self, state: TileConfig, want: TileConfig, knob: str):
+        """Compiled configs of ``want``'s variant with its ``knob`` (or, of the LDS stages, any more or any fewer than
+        ``state`` has, as in ``want``), the nearest first; raster height and K split as in ``want``, or unsplit where
+        the variant takes no such split."""
+        def distance(c: TileConfig) -> float:
+            return abs(c.lds_stages - want.lds_stages) + sum(
+                abs(math.log2(getattr(c, k) / getattr(want, k))) for k in ("block_m", "block_n", "block_k", "waves"))
+
+        def moved(c: TileConfig) -> bool:
+            if knob == "lds_stages":
+                return (c.lds_stages - state.lds_stages) * (want.lds_stages - state.lds_stages) > 0
+            return getattr(c, knob) == getattr(want, knob)
+
+        for c in sorted((c for c in self._compiled if c.variant == want.variant and moved(c)), key=distance):
+            for parts in dict.fromkeys((want.split_k, 1)):
+                yield replace(c, group_m=want.group_m, split_k=parts)
 
     def legal_actions(self, state: TileConfig) -> list[Atom]:
         out = []
