@@ -16,7 +16,7 @@
 //
 // Nothing is kept between calls but the shapes' configs: no pointer, tensor
 // or identity.  The GIL is held throughout except around the launch, as
-// ctypes does, so the table needs no lock.
+// ctypes does, so the table needs no lock; nothing shared is read there.
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
@@ -153,13 +153,14 @@ PyObject* call(PyObject*, PyObject* const* args, Py_ssize_t n) {
     void* stream = (void*)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).stream();
     const void *ap = a->data_ptr(), *bp = b->data_ptr(), *gp = g ? g->data_ptr() : nullptr;
     void* op = given->data_ptr();
+    // The entry point is read before the GIL is given up: another thread's
+    // bind() may then put another library's in its place.
+    const MatmulFn mm = kind == kLhs ? g_lib.lhs : kind == kLhsTF32 ? g_lib.lhsT_f32 : g_lib.lhsT_bf16;
+    const RmsFn rms = g_lib.rms;
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    if (kind == kRms || kind == kRmsNoGamma)
-      rc = g_lib.rms(ap, gp, bp, op, (int)M, (int)N, (int)K, eps, &cfg, stream);
-    else
-      rc = (kind == kLhs ? g_lib.lhs : kind == kLhsTF32 ? g_lib.lhsT_f32 : g_lib.lhsT_bf16)(ap, bp, op, (int)M, (int)N,
-                                                                                           (int)K, &cfg, stream);
+    if (kind == kRms || kind == kRmsNoGamma) rc = rms(ap, gp, bp, op, (int)M, (int)N, (int)K, eps, &cfg, stream);
+    else rc = mm(ap, bp, op, (int)M, (int)N, (int)K, &cfg, stream);
     Py_END_ALLOW_THREADS
     if (rc != 0) {
       static const char* const names[] = {"matmul_lhsT_rhs", "matmul_lhsT_rhs_f32", "rmsnorm_matmul", "matmul_lhs_rhs",
