@@ -183,20 +183,28 @@ PyObject* call(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 // bind(env, lhsT_bf16, lhsT_f32, rms, lhs, check_rc): the library's entry
 // points (addresses), the value of MI_KERNELS_LIB they were found with, and
-// the function that raises a return code's error.
+// the function that raises a return code's error.  Another library than the
+// bound one drops every shape's config.
 PyObject* bind(PyObject*, PyObject* args) {
   const char* env;
   unsigned long long p0, p1, p2, p3;
   PyObject* check_rc;
   if (!PyArg_ParseTuple(args, "sKKKKO", &env, &p0, &p1, &p2, &p3, &check_rc)) return nullptr;
-  Py_INCREF(check_rc);
-  Py_XDECREF(g_lib.check_rc);
+  const MatmulFn lhsT_bf16 = (MatmulFn)(uintptr_t)p0, lhsT_f32 = (MatmulFn)(uintptr_t)p1, lhs = (MatmulFn)(uintptr_t)p3;
+  const RmsFn rms = (RmsFn)(uintptr_t)p2;
+  // The shapes' configs are the bound library's own.
+  if (g_lib.env != env || g_lib.lhsT_bf16 != lhsT_bf16 || g_lib.lhsT_f32 != lhsT_f32 || g_lib.rms != rms ||
+      g_lib.lhs != lhs)
+    g_configs.clear();
   g_lib.env = env;
-  g_lib.lhsT_bf16 = (MatmulFn)(uintptr_t)p0;
-  g_lib.lhsT_f32 = (MatmulFn)(uintptr_t)p1;
-  g_lib.rms = (RmsFn)(uintptr_t)p2;
-  g_lib.lhs = (MatmulFn)(uintptr_t)p3;
+  g_lib.lhsT_bf16 = lhsT_bf16;
+  g_lib.lhsT_f32 = lhsT_f32;
+  g_lib.rms = rms;
+  g_lib.lhs = lhs;
+  Py_INCREF(check_rc);
+  PyObject* const before = g_lib.check_rc;
   g_lib.check_rc = check_rc;
+  Py_XDECREF(before);
   Py_RETURN_NONE;
 }
 

@@ -13,6 +13,7 @@ from __future__ import annotations
 import ctypes
 import itertools
 import json
+import os
 from dataclasses import asdict, dataclass, replace
 from pathlib import Path
 
@@ -211,9 +212,10 @@ def default_config(func_name: str, M: int, N: int, K: int) -> TileConfig:
     ``rmsnorm_matmul_online`` (the fused product without gamma) takes its own
     tuned entry, else the gamma one, else ``mi_default_config_no_gamma``.
 
-    Memoised per (name, shape) until the tuned table is reloaded: a call
-    without a config pays a dict lookup, not a table scan and a library call."""
-    key = (func_name, M, N, K)
+    Memoised per (name, shape, library) until the tuned table is reloaded: a
+    call without a config pays a dict lookup, not a table scan and a library
+    call."""
+    key = (func_name, M, N, K, os.environ.get("MI_KERNELS_LIB"))
     cfg = _DEFAULT_CACHE.get(key)
     if cfg is not None:
         return cfg
