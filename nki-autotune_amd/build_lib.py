@@ -23,6 +23,7 @@ import subprocess
 import sys
 import sysconfig
 from concurrent.futures import ThreadPoolExecutor
+from importlib import metadata
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
@@ -88,10 +89,15 @@ def _link(objs: list[Path], lib: Path) -> None:
 
 
 def _build_torch_call(force: bool) -> None:
-    """csrc/host/mi_torch_call.cpp -> kernel_library/_torch_call.so (g++ against the installed torch)."""
+    """csrc/host/mi_torch_call.cpp -> kernel_library/_torch_call.so (g++ against the installed torch).
+
+    Built again when a source is newer, or when it was built for another torch or Python than the running ones."""
     src = CSRC / "host" / "mi_torch_call.cpp"
     deps = [src, *INCLUDE.glob("*.h")]
-    if not force and TORCH_CALL.exists() and TORCH_CALL.stat().st_mtime >= max(p.stat().st_mtime for p in deps):
+    stamp = BUILD / "torch_call.for"
+    built_for = f"torch {metadata.version('torch')}, Python {sys.version.split()[0]}"
+    if (not force and TORCH_CALL.exists() and stamp.exists() and stamp.read_text() == built_for
+            and TORCH_CALL.stat().st_mtime >= max(p.stat().st_mtime for p in deps)):
         return
     import torch
     from torch.utils import cpp_extension
@@ -107,6 +113,7 @@ def _build_torch_call(force: bool) -> None:
     if proc.returncode != 0:
         raise RuntimeError(f"g++ failed for {src.name}:\n{proc.stdout}{proc.stderr}")
     os.replace(tmp, TORCH_CALL)
+    stamp.write_text(built_for)
 
 
 def build(jobs: int | None = None, force: bool = False, verbose: bool = False) -> Path:

@@ -26,10 +26,12 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include <climits>
 #include <cstdint>
 #include <cstdlib>
+#include <cstring>
 #include <string>
 #include <unordered_map>
 
@@ -235,4 +237,18 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_torch_call", nullptr, -1, kMetho
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__torch_call() { return PyModule_Create(&kModule); }
+// Built against one torch's headers, so it loads beside that torch only (the
+// Python body then serves the calls).
+PyMODINIT_FUNC PyInit__torch_call() {
+  PyObject* torch = PyImport_ImportModule("torch");
+  if (!torch) return nullptr;
+  PyObject* version = PyObject_GetAttrString(torch, "__version__");
+  Py_DECREF(torch);
+  if (!version) return nullptr;
+  const char* now = PyUnicode_AsUTF8(version);
+  const size_t n = std::strlen(TORCH_VERSION);
+  const bool same = now && std::strncmp(now, TORCH_VERSION, n) == 0 && (now[n] == '\0' || now[n] == '+');
+  if (now && !same) PyErr_Format(PyExc_ImportError, "built for torch %s, found %s", TORCH_VERSION, now);
+  Py_DECREF(version);
+  return same ? PyModule_Create(&kModule) : nullptr;
+}

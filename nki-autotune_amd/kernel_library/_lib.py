@@ -8,7 +8,9 @@ kernel of this package.
 from __future__ import annotations
 
 import ctypes
+import importlib
 import os
+import warnings
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "libmi_kernels.so"
@@ -161,6 +163,24 @@ def load(path: str | os.PathLike) -> ctypes.CDLL:
 def lib() -> ctypes.CDLL:
     """Load (once) and return libmi_kernels.so; raise if it was never built."""
     return load(os.environ.get("MI_KERNELS_LIB", LIB_PATH))
+
+
+def torch_call():
+    """The native half of a call without a config: the ``_torch_call`` extension, or, where it cannot be imported, a
+    stand-in that leaves every call to the Python body.
+
+    A tree that is not built has neither the extension nor libmi_kernels.so and imports all the same: its first call
+    raises with the build command.  A built one whose extension does not load (built for another torch or Python)
+    says so once, as each call then takes 7 us more host time."""
+    import torch  # noqa: F401  (loads the libraries that the extension links)
+
+    try:
+        return importlib.import_module("kernel_library._torch_call")
+    except ImportError as exc:
+        if LIB_PATH.exists():
+            warnings.warn(f"the native call extension does not load ({exc}); calls go through Python until it is built "
+                          "again with `python nki-autotune_amd/build_lib.py`", RuntimeWarning, stacklevel=2)
+        return importlib.import_module("kernel_library._torch_call_none")
 
 
 def last_error() -> str:

@@ -1,0 +1,24 @@
+"""Stands in for the ``_torch_call`` extension where it cannot be imported.
+
+The extension is the native half of a call without a config
+(csrc/host/mi_torch_call.cpp); the Python body of every operation serves all
+calls without it, at more host time per call.  Nothing is remembered here,
+and every call is left to the Python body, as the extension leaves those it
+does not know.
+"""
+
+
+def call(kind, a, b, gamma, eps, out):
+    return None
+
+
+def bind(env, lhsT_bf16, lhsT_f32, rms, lhs, check_rc):
+    return None
+
+
+def remember(*shape_and_config):
+    return None
+
+
+def forget():
+    return None

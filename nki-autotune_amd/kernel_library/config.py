@@ -17,9 +17,9 @@ import os
 from dataclasses import asdict, dataclass, replace
 from pathlib import Path
 
-import torch  # noqa: F401  (loads the libraries that _torch_call links)
+from kernel_library import _lib
 
-from kernel_library import _lib, _torch_call
+_torch_call = _lib.torch_call()
 
 KERNEL_IDS = {
     "matmul_lhsT_rhs": _lib.MI_KERNEL_MATMUL_LHST_RHS_BF16,

@@ -32,8 +32,8 @@ import os
 
 import torch
 
-from kernel_library import _lib, _torch_call
-from kernel_library.config import TileConfig, default_config
+from kernel_library import _lib
+from kernel_library.config import TileConfig, _torch_call, default_config
 
 EPS = 1e-6
 
