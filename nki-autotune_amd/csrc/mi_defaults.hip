@@ -5,6 +5,7 @@
 // shapes, and studies of 83 shapes and of seeded random ones.  Host code
 // only.
 #include <math.h>
+#include <stdint.h>
 
 #include "mi_capi_internal.hpp"
 
@@ -608,7 +609,9 @@ mi_tile_cfg faster_of(int kernel_id, const Timed* table, int n, const Timed& old
   double best_t = margin * fitted_time(old, pick.split_k, M, N, K);
   mi_tile_cfg best = pick;
   for (int i = 0; i < n; ++i) {
+    const long long tiles = tiles_of(M, N, table[i].c.block_m, table[i].c.block_n);
     for (const int parts : {1, 2, 3, 4, 5, 6, 7, 8, 12, 16}) {
+      if (parts > 1 && tiles * parts > kCUs) break;  // runs_split refuses it and every larger one
       const double t = fitted_time(table[i], parts, M, N, K);
       if (t < best_t && runs_split(kernel_id, table[i].c, parts, M, N, K)) {
         best_t = t;
@@ -755,32 +758,25 @@ mi_tile_cfg refined_fused(int M, int N, int K) {
                  M, N, K);
 }
 
-}  // namespace
-
-// The library default: the estimates and rules above, fitted to timed
-// campaigns and checked against full autotune sweeps.
-int pick_default(int kernel_id, int M, int N, int K, mi_tile_cfg* cfg) {
+// The estimates and rules above, fitted to timed campaigns and checked
+// against full autotune sweeps.
+mi_tile_cfg estimated_default(int kernel_id, int M, int N, int K) {
   const bool lhs = kernel_id == MI_KERNEL_MATMUL_LHS_RHS_BF16;
   switch (kernel_id) {
     case MI_KERNEL_MATMUL_LHST_RHS_F32:
-      *cfg = f32_default(M, N, K);
-      break;
+      return f32_default(M, N, K);
     case MI_KERNEL_MATMUL_LHST_RHS_BF16:
     case MI_KERNEL_MATMUL_LHS_RHS_BF16:
-      *cfg = M <= 128 ? refined_skinny(kernel_id, M, N, K) : refined_matmul(kernel_id, lhs, M, N, K);
-      break;
+      return M <= 128 ? refined_skinny(kernel_id, M, N, K) : refined_matmul(kernel_id, lhs, M, N, K);
     case MI_KERNEL_RMSNORM_MATMUL_BF16:
-      *cfg = M <= 128 ? refined_skinny(kernel_id, M, N, K) : refined_fused(M, N, K);
-      break;
+      return M <= 128 ? refined_skinny(kernel_id, M, N, K) : refined_fused(M, N, K);
     default:
-      *cfg = {256, 256, 64, 8, 2, 1, 8, 0};
-      break;
+      return {256, 256, 64, 8, 2, 1, 8, 0};
   }
-  return MI_OK;
 }
 
-// The fused kernel's default for a call without gamma: pick_default's
-// choice, except that its 128x128, 64x128 and 64x64 blocks (split or not) at
+// The fused kernel's default for a call without gamma: the choice with
+// gamma, except that its 128x128, 64x128 and 64x64 blocks (split or not) at
 // M > 128 give way to a gamma-free variant, unsplit, where that is faster by
 // the fitted times: 64x128 and 64x64 to variant 14 with the same block,
 // 128x128 to variant 16 at 128x128 or variant 14 at 64x128 or 64x64.  At 50
@@ -794,19 +790,18 @@ int pick_default(int kernel_id, int M, int N, int K, mi_tile_cfg* cfg) {
 // 512x4096x4096 (128 tiles); 10.1 / 7.9 / 6.4 at 1024^3 (64 tiles).  The
 // larger blocks (128x512, 256x256 two-pass, 128x256) stay, variant 14 being
 // 0-8 % slower there.  Skinny M keeps its non-temporal variants.
-int pick_default_no_gamma(int M, int N, int K, mi_tile_cfg* cfg) {
-  const int rc = pick_default(MI_KERNEL_RMSNORM_MATMUL_BF16, M, N, K, cfg);
-  if (rc != MI_OK) return rc;
-  const int v = cfg->variant, bm = cfg->block_m, bn = cfg->block_n;
+mi_tile_cfg estimated_no_gamma(int M, int N, int K) {
+  const mi_tile_cfg c = estimated_default(MI_KERNEL_RMSNORM_MATMUL_BF16, M, N, K);
+  const int v = c.variant, bm = c.block_m, bn = c.block_n;
   const bool one_pass_or_two = v == 4 || v == 5 || v == 13 || v == 15;
   const bool small_block = (bm == 128 && bn == 128) || (bm == 64 && bn == 128) || (bm == 64 && bn == 64);
-  if (M <= 128 || !one_pass_or_two || !small_block) return MI_OK;
+  if (M <= 128 || !one_pass_or_two || !small_block) return c;
   const mi_tile_cfg free[] = {{128, 128, 32, 4, 4, 1, 8, 16}, {64, 128, 64, 4, 4, 1, 8, 14}, {64, 64, 64, 4, 4, 1, 8, 14}};
   const long long t128 = tiles_of(M, N, 128, 128);
   int pick = bm == 128 ? (2 * t128 > kCUs ? 0 : 4 * t128 > kCUs ? 1 : 2) : bn == 128 ? 1 : 2;
-  const Timed* old = timed(kNoGammaTimed, count(kNoGammaTimed), *cfg);
+  const Timed* old = timed(kNoGammaTimed, count(kNoGammaTimed), c);
   if (old) {
-    double best_t = fitted_time(*old, cfg->split_k, M, N, K);
+    double best_t = fitted_time(*old, c.split_k, M, N, K);
     pick = -1;
     for (int i = 0; i < 3; ++i) {
       if (bm != 128 && (free[i].block_m != bm || free[i].block_n != bn)) continue;
@@ -817,12 +812,42 @@ int pick_default_no_gamma(int M, int N, int K, mi_tile_cfg* cfg) {
       }
     }
   }
-  if (pick >= 0) {
-    const int group_m = cfg->group_m;
-    *cfg = free[pick];
-    cfg->group_m = group_m;
-  }
+  if (pick < 0) return c;
+  mi_tile_cfg picked = free[pick];
+  picked.group_m = c.group_m;
+  return picked;
+}
+
+// The picks of the shapes that a thread calls in turn.  An estimate takes up
+// to 1 us of host time (0.27 at lhsT 2048x1024x8192) beside a launch's 2.8,
+// and a program calls few shapes many times; one found here costs 0.006 us.
+// One slot per hash, so at most kPicks per thread (12 KB), without a lock.
+struct Pick {
+  int kind;  // kernel id + 1, or kNoGamma; 0: empty
+  int M, N, K;
+  mi_tile_cfg cfg;
+};
+constexpr int kPickBits = 8, kPicks = 1 << kPickBits, kNoGamma = MI_NUM_KERNELS + 1;
+thread_local Pick t_picks[kPicks];
+
+template <class F>
+int picked(int kind, int M, int N, int K, mi_tile_cfg* cfg, F&& estimate) {
+  uint64_t h = (uint64_t)kind;
+  for (const int v : {M, N, K}) h = (h ^ (uint32_t)v) * 0x9E3779B97F4A7C15ull;
+  Pick& p = t_picks[h >> (64 - kPickBits)];
+  if (p.kind != kind || p.M != M || p.N != N || p.K != K) p = Pick{kind, M, N, K, estimate()};
+  *cfg = p.cfg;
   return MI_OK;
+}
+
+}  // namespace
+
+int pick_default(int kernel_id, int M, int N, int K, mi_tile_cfg* cfg) {
+  return picked(kernel_id + 1, M, N, K, cfg, [=] { return estimated_default(kernel_id, M, N, K); });
+}
+
+int pick_default_no_gamma(int M, int N, int K, mi_tile_cfg* cfg) {
+  return picked(kNoGamma, M, N, K, cfg, [=] { return estimated_no_gamma(M, N, K); });
 }
 
 }  // namespace capi
