@@ -775,47 +775,76 @@ mi_tile_cfg estimated_default(int kernel_id, int M, int N, int K) {
   }
 }
 
-// The fused kernel's default for a call without gamma: the choice with
-// gamma, except that its 128x128, 64x128 and 64x64 blocks (split or not) at
-// M > 128 give way to a gamma-free variant, unsplit, where that is faster by
-// the fitted times: 64x128 and 64x64 to variant 14 with the same block,
-// 128x128 to variant 16 at 128x128 or variant 14 at 64x128 or 64x64.  At 50
-// shapes drawn afterwards the pick ran within 1.035 of the fastest on
-// average, against 1.16 at 40 for always taking the gamma-free variant (152x160x5112, where 64x64 blocks unsplit leave 247 CUs idle: 23.3 ->
-// 9 us in 16 parts; 872x280x9560: 45 -> 21 us).  A pick that was not timed
-// without gamma moves as those rules did: a 128 x 128 block to the largest
-// block whose grid keeps more than half the CUs busy.  Measured without
-// gamma (us, 128 x 128 v16 / 64 x 128 v14 / 64 x 64 v14): 59.9 / 76.1 / 75.5
-// at 384x8192x8192 (192 tiles of 128 x 128); 29.2 / 23.5 / 28.7 at
-// 512x4096x4096 (128 tiles); 10.1 / 7.9 / 6.4 at 1024^3 (64 tiles).  The
-// larger blocks (128x512, 256x256 two-pass, 128x256) stay, variant 14 being
-// 0-8 % slower there.  Skinny M keeps its non-temporal variants.
-mi_tile_cfg estimated_no_gamma(int M, int N, int K) {
-  const mi_tile_cfg c = estimated_default(MI_KERNEL_RMSNORM_MATMUL_BF16, M, N, K);
-  const int v = c.variant, bm = c.block_m, bn = c.block_n;
-  const bool one_pass_or_two = v == 4 || v == 5 || v == 13 || v == 15;
-  const bool small_block = (bm == 128 && bn == 128) || (bm == 64 && bn == 128) || (bm == 64 && bn == 64);
-  if (M <= 128 || !one_pass_or_two || !small_block) return c;
-  const mi_tile_cfg free[] = {{128, 128, 32, 4, 4, 1, 8, 16}, {64, 128, 64, 4, 4, 1, 8, 14}, {64, 64, 64, 4, 4, 1, 8, 14}};
+// The fused kernel's default for a call without gamma: the rules' choice,
+// its 128x128, 64x128 and 64x64 blocks (split or not) at M > 128 given to a
+// gamma-free variant, unsplit: 64x128 and 64x64 to variant 14 with the same
+// block, 128x128 to the largest block whose grid keeps more than half the
+// CUs busy, variant 16 at 128x128 or variant 14 at 64x128 or 64x64.
+// Measured without gamma (us, 128 x 128 v16 / 64 x 128 v14 / 64 x 64 v14):
+// 59.9 / 76.1 / 75.5 at 384x8192x8192 (192 tiles of 128 x 128);
+// 29.2 / 23.5 / 28.7 at 512x4096x4096 (128 tiles); 10.1 / 7.9 / 6.4 at
+// 1024^3 (64 tiles).  The larger blocks (128x512, 256x256 two-pass, 128x256)
+// stay, variant 14 being 0-8 % slower there.  Skinny M keeps its
+// non-temporal variants.
+const mi_tile_cfg kGammaFree[] = {
+    {128, 128, 32, 4, 4, 1, 8, 16}, {64, 128, 64, 4, 4, 1, 8, 14}, {64, 64, 64, 4, 4, 1, 8, 14}};
+
+bool small_one_or_two_pass(const mi_tile_cfg& c) {
+  const bool one_pass_or_two = c.variant == 4 || c.variant == 5 || c.variant == 13 || c.variant == 15;
+  return one_pass_or_two && ((c.block_m == 128 && c.block_n == 128) || (c.block_m == 64 && c.block_n == 128) ||
+                             (c.block_m == 64 && c.block_n == 64));
+}
+
+mi_tile_cfg no_gamma_default(int M, int N, int K) {
+  const mi_tile_cfg c = fused_default(M, N, K);
+  if (M <= 128 || !small_one_or_two_pass(c)) return c;
   const long long t128 = tiles_of(M, N, 128, 128);
-  int pick = bm == 128 ? (2 * t128 > kCUs ? 0 : 4 * t128 > kCUs ? 1 : 2) : bn == 128 ? 1 : 2;
-  const Timed* old = timed(kNoGammaTimed, count(kNoGammaTimed), c);
-  if (old) {
-    double best_t = fitted_time(*old, c.split_k, M, N, K);
-    pick = -1;
-    for (int i = 0; i < 3; ++i) {
-      if (bm != 128 && (free[i].block_m != bm || free[i].block_n != bn)) continue;
-      const double t = fitted_time(*timed(kNoGammaTimed, count(kNoGammaTimed), free[i]), 1, M, N, K);
+  mi_tile_cfg free = kGammaFree[c.block_m == 128 ? (2 * t128 > kCUs ? 0 : 4 * t128 > kCUs ? 1 : 2) : c.block_n == 128 ? 1 : 2];
+  free.group_m = c.group_m;
+  return free;
+}
+
+// The refined choice with gamma, its small block split or as the gamma-free
+// variant of the same size (128x128 also of the smaller ones) where the
+// times fitted without gamma say that is faster: 152x160x5112, where 64x64
+// blocks unsplit leave 247 CUs idle, 23.3 -> 9 us in 16 parts; 872x280x9560
+// 45 -> 21 us.  The choice above stays where the times fitted without gamma
+// say it is faster (by 5 %; by 15 % where the refined one is a small block,
+// whose short splits those times know to no better), and, timed itself,
+// before a block that was not: without gamma 256 x 128 variant 5 ran 1.2-1.4
+// x the gamma-free variants' time (12936x16x8400 48 -> 61 us) and, below
+// K = 512, 1.03-1.2 x that of 128 x 256.  At 996 drawn shapes past skinny M,
+// inside and outside the fitted sizes, whose refined choice is another, this
+// is 1.47 x faster than the choice above on average and over 3 % slower at
+// 19; the refined choice everywhere was so at 106, to 5.3 x (264x880x122680,
+// whose 64x64 split became the gamma-free block unsplit: 155 -> 821 us).
+// Skinny M takes the refined choice where either splits K (1.12 x over 215
+// shapes): both unsplit, the cached blocks that win with gamma lose to the
+// non-temporal ones without it (24x5752x320: 4.0 -> 4.25 us).
+mi_tile_cfg estimated_no_gamma(int M, int N, int K) {
+  const mi_tile_cfg rules = no_gamma_default(M, N, K);
+  mi_tile_cfg c = estimated_default(MI_KERNEL_RMSNORM_MATMUL_BF16, M, N, K);
+  if (M <= 128) return c.split_k > 1 || rules.split_k > 1 ? c : rules;
+  constexpr int n = count(kNoGammaTimed);
+  const Timed *by_rules = timed(kNoGammaTimed, n, rules), *refined_one = timed(kNoGammaTimed, n, c);
+  if (!refined_one) return by_rules && (rules.variant == 14 || rules.variant == 16 || K < 512) ? rules : c;
+  const bool small = small_one_or_two_pass(c);
+  double best_t = fitted_time(*refined_one, c.split_k, M, N, K);
+  if (small) {
+    const int bm = c.block_m, bn = c.block_n;
+    for (const mi_tile_cfg& free : kGammaFree) {
+      if (bm != 128 && (free.block_m != bm || free.block_n != bn)) continue;
+      const double t = fitted_time(*timed(kNoGammaTimed, n, free), 1, M, N, K);
       if (t < best_t) {
         best_t = t;
-        pick = i;
+        c = free;
       }
     }
+  } else if (c.split_k > 1) {
+    return c;  // 1.02-1.6 x faster than the choice above at 10 of 12 such shapes, 0.94 at the others
   }
-  if (pick < 0) return c;
-  mi_tile_cfg picked = free[pick];
-  picked.group_m = c.group_m;
-  return picked;
+  if (!by_rules) return c;
+  return best_t > (small ? 1.15 : 1.05) * fitted_time(*by_rules, rules.split_k, M, N, K) ? rules : c;
 }
 
 // The picks of the shapes that a thread calls in turn.  An estimate takes up

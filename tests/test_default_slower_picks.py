@@ -1,0 +1,45 @@
+"""Default picks at shapes where a block was timed slower than another one that the rules offer: not the slower block.
+
+Each entry: the shape, the slower block, and the times (us, calls back to back in interleaved rounds over three sets of
+inputs) of that block and of the faster one.
+"""
+
+import ctypes
+
+import pytest
+
+from kernel_library import _lib
+from kernel_library.config import TileConfig
+
+LHST, F32, FUSED, LHS, NO_GAMMA = range(5)
+
+SLOWER = [
+    # Without gamma: the gamma default's block, or its gamma-free form, behind the gamma-free choice of the rules.
+    (NO_GAMMA, (264, 880, 122680), "bm64_bn64_bk64_w4_s4_v14", 821, 155),
+    (NO_GAMMA, (208, 2264, 22400), "bm64_bn64_bk64_w4_s4_v14", 106, 58.7),
+    (NO_GAMMA, (3808, 128, 2288), "bm64_bn128_bk64_w4_s4_v5_k4", 14.5, 10.3),
+    (NO_GAMMA, (9824, 16, 5624), "bm256_bn128_bk32_w8_s3_v5_k4", 43.5, 31.7),
+    (NO_GAMMA, (12936, 16, 8400), "bm256_bn128_bk32_w8_s3_v5_k4", 61.5, 48.0),
+    (NO_GAMMA, (16928, 800, 1848), "bm256_bn128_bk32_w8_s3_v5", 87.0, 71.8),
+    (NO_GAMMA, (60984, 208, 8), "bm256_bn128_bk32_w8_s3_v5", 10.6, 8.9),
+    (NO_GAMMA, (3016, 7208, 168), "bm128_bn512_bk32_w8_s3_v4", 22.1, 20.6),
+    (NO_GAMMA, (24, 5752, 320), "bm32_bn128_bk64_w4_s4_v5", 4.25, 3.98),
+    (NO_GAMMA, (32, 44944, 80), "bm32_bn128_bk64_w4_s4_v5", 6.4, 5.05),
+    (NO_GAMMA, (64, 37360, 16), "bm64_bn128_bk64_w4_s4_v5", 7.0, 5.4),
+]
+
+
+def _default(kind, M, N, K):
+    c = _lib.MiTileCfg()
+    L = _lib.lib()
+    rc = L.mi_default_config_no_gamma(M, N, K, ctypes.byref(c)) if kind == NO_GAMMA else \
+        L.mi_default_config(kind, M, N, K, ctypes.byref(c))
+    assert rc == _lib.MI_OK
+    return TileConfig.from_c(c)
+
+
+@pytest.mark.parametrize("kind,shape,slower,slow_us,fast_us", SLOWER)
+def test_the_slower_block_is_not_picked(kind, shape, slower, slow_us, fast_us):
+    assert fast_us < 0.95 * slow_us
+    TileConfig.from_name(slower)
+    assert _default(kind, *shape).name != slower
