@@ -606,9 +606,18 @@ bool runs_split(int kernel_id, const mi_tile_cfg& c, int parts, int M, int N, in
 // with the least fitted time where that is under `margin` of the pick's own.
 mi_tile_cfg faster_of(int kernel_id, const Timed* table, int n, const Timed& old, const mi_tile_cfg& pick, double margin,
                       int M, int N, int K) {
+  // The fit reads x once.  Past the L2s (64 MiB of x) every column of tiles
+  // of the fused kernel reads it again, so where the pick spans the columns
+  // with one tile, its place is for blocks that do as well (us, 128 x 512 in
+  // 4 parts against 128-wide blocks, three columns of them: 110 against 126
+  // at 7168x328x14688, 70 against 85 at 5088x336x9936, 87 against 112 at
+  // 4376x312x13424; at 61 MiB, 2520x336x12688, 47 against 43).
+  const bool one_column =
+      kernel_id == MI_KERNEL_RMSNORM_MATMUL_BF16 && N <= pick.block_n && (long long)M * K * 2 > (64LL << 20);
   double best_t = margin * fitted_time(old, pick.split_k, M, N, K);
   mi_tile_cfg best = pick;
   for (int i = 0; i < n; ++i) {
+    if (one_column && N > table[i].c.block_n) continue;
     const long long tiles = tiles_of(M, N, table[i].c.block_m, table[i].c.block_n);
     for (const int parts : {1, 2, 3, 4, 5, 6, 7, 8, 12, 16}) {
       if (parts > 1 && tiles * parts > kCUs) break;  // runs_split refuses it and every larger one

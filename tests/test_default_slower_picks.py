@@ -26,6 +26,13 @@ SLOWER = [
     (NO_GAMMA, (24, 5752, 320), "bm32_bn128_bk64_w4_s4_v5", 4.25, 3.98),
     (NO_GAMMA, (32, 44944, 80), "bm32_bn128_bk64_w4_s4_v5", 6.4, 5.05),
     (NO_GAMMA, (64, 37360, 16), "bm64_bn128_bk64_w4_s4_v5", 7.0, 5.4),
+    # Three columns of tiles where one spans the output, with an x that no cache holds.
+    (FUSED, (7168, 328, 14688), "bm256_bn128_bk32_w8_s3_v5_k3", 126.0, 110.1),
+    (FUSED, (5368, 304, 8456), "bm256_bn128_bk32_w8_s3_v5_k4", 70.6, 62.6),
+    (FUSED, (4464, 272, 10120), "bm256_bn128_bk32_w8_s3_v5_k4", 75.2, 66.9),
+    (FUSED, (2664, 336, 15392), "bm128_bn128_bk32_w4_s4_v5_k4", 60.8, 56.6),
+    (NO_GAMMA, (1536, 264, 50216), "bm256_bn128_bk32_w8_s3_v5_k12", 125.3, 90.5),
+    (NO_GAMMA, (7032, 352, 13096), "bm256_bn128_bk32_w8_s3_v5_k3", 134.4, 101.4),
 ]
 
 
