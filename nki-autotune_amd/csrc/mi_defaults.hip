@@ -614,10 +614,24 @@ mi_tile_cfg faster_of(int kernel_id, const Timed* table, int n, const Timed& old
   // 4376x312x13424; at 61 MiB, 2520x336x12688, 47 against 43).
   const bool one_column =
       kernel_id == MI_KERNEL_RMSNORM_MATMUL_BF16 && N <= pick.block_n && (long long)M * K * 2 > (64LL << 20);
+  // Below K = 512 a matmul past skinny M is bound by its output's stores,
+  // which the fits know only as a part of each tile; they then take blocks
+  // too small.  lhsT.rhs in 256 x 256 blocks stays there (256 x 128 in their
+  // place was over 3 % slower at 30 of 106 shapes, 128 x 256 at 26 of 94: us,
+  // 51 -> 59 at 4072x14904x176, 77 -> 86 at 3496x26040x168, 316 -> 407 at
+  // 1224x244688x312).  lhs.rhs takes no 256 x 128 (6 of 14), and 128 x 128
+  // only in the place of a 128-wide block (21 of 48 of another width; 7.4 ->
+  // 8.1 at 46328x192x8).
+  const bool short_k = K < 512 && M > 128;
+  const bool lhs = kernel_id == MI_KERNEL_MATMUL_LHS_RHS_BF16, lhsT = kernel_id == MI_KERNEL_MATMUL_LHST_RHS_BF16;
+  if (short_k && lhsT && pick.block_m == 256 && pick.block_n == 256) return pick;
   double best_t = margin * fitted_time(old, pick.split_k, M, N, K);
   mi_tile_cfg best = pick;
   for (int i = 0; i < n; ++i) {
     if (one_column && N > table[i].c.block_n) continue;
+    if (short_k && lhs && table[i].c.block_n == 128 &&
+        (table[i].c.block_m == 256 || (table[i].c.block_m == 128 && pick.block_n != 128)))
+      continue;
     const long long tiles = tiles_of(M, N, table[i].c.block_m, table[i].c.block_n);
     for (const int parts : {1, 2, 3, 4, 5, 6, 7, 8, 12, 16}) {
       if (parts > 1 && tiles * parts > kCUs) break;  // runs_split refuses it and every larger one

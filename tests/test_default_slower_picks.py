@@ -33,6 +33,15 @@ SLOWER = [
     (FUSED, (2664, 336, 15392), "bm128_bn128_bk32_w4_s4_v5_k4", 60.8, 56.6),
     (NO_GAMMA, (1536, 264, 50216), "bm256_bn128_bk32_w8_s3_v5_k12", 125.3, 90.5),
     (NO_GAMMA, (7032, 352, 13096), "bm256_bn128_bk32_w8_s3_v5_k3", 134.4, 101.4),
+    # Short K, the output's stores its bound: smaller blocks.
+    (LHST, (4072, 14904, 176), "bm256_bn128_bk32_w4_s3_v1", 59.3, 51.4),
+    (LHST, (3496, 26040, 168), "bm256_bn128_bk32_w4_s3_v1", 85.9, 76.9),
+    (LHST, (1224, 244688, 312), "bm128_bn256_bk32_w4_s3_v1", 407.0, 316.0),
+    (LHST, (1240, 158800, 368), "bm256_bn128_bk32_w4_s3_v1", 267.0, 218.7),
+    (LHS, (65344, 120, 344), "bm256_bn128_bk64_w8_s3", 15.2, 13.2),
+    (LHS, (4832, 1648, 456), "bm256_bn128_bk64_w8_s3", 14.4, 13.5),
+    (LHS, (400, 53104, 16), "bm128_bn128_bk32_w4_s4_v1", 15.1, 12.9),
+    (LHS, (46328, 192, 8), "bm128_bn128_bk32_w4_s4_v1", 8.1, 7.4),
 ]
 
 
@@ -47,6 +56,6 @@ def _default(kind, M, N, K):
 
 @pytest.mark.parametrize("kind,shape,slower,slow_us,fast_us", SLOWER)
 def test_the_slower_block_is_not_picked(kind, shape, slower, slow_us, fast_us):
-    assert fast_us < 0.95 * slow_us
+    assert fast_us < 0.96 * slow_us
     TileConfig.from_name(slower)
     assert _default(kind, *shape).name != slower
