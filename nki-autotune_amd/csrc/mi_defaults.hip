@@ -624,6 +624,12 @@ mi_tile_cfg faster_of(int kernel_id, const Timed* table, int n, const Timed& old
   // 8.1 at 46328x192x8).
   const bool short_k = K < 512 && M > 128;
   const bool lhs = kernel_id == MI_KERNEL_MATMUL_LHS_RHS_BF16, lhsT = kernel_id == MI_KERNEL_MATMUL_LHST_RHS_BF16;
+  // Skinny, a split of the rules' stays one past K = 2048, where one
+  // workgroup's chain over all of K is longer than the fits say: unsplit in
+  // its place ran 0.77-1.0 x as fast on lhsT.rhs (112x752x2288 8.6 -> 11.3
+  // us; 1.28 x faster at 63 shapes with K 1300-1900) and 0.84-1.1 x on lhs.rhs
+  // (80x5928x2224 17.3 -> 20.6; 1.35 x faster at 60).
+  const bool stays_split = M <= 128 && (lhs || lhsT) && pick.split_k > 1 && K > 2048;
   if (short_k && lhsT && pick.block_m == 256 && pick.block_n == 256) return pick;
   double best_t = margin * fitted_time(old, pick.split_k, M, N, K);
   mi_tile_cfg best = pick;
@@ -635,6 +641,7 @@ mi_tile_cfg faster_of(int kernel_id, const Timed* table, int n, const Timed& old
     const long long tiles = tiles_of(M, N, table[i].c.block_m, table[i].c.block_n);
     for (const int parts : {1, 2, 3, 4, 5, 6, 7, 8, 12, 16}) {
       if (parts > 1 && tiles * parts > kCUs) break;  // runs_split refuses it and every larger one
+      if (parts == 1 && stays_split) continue;
       const double t = fitted_time(table[i], parts, M, N, K);
       if (t < best_t && runs_split(kernel_id, table[i].c, parts, M, N, K)) {
         best_t = t;

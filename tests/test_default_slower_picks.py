@@ -42,6 +42,12 @@ SLOWER = [
     (LHS, (4832, 1648, 456), "bm256_bn128_bk64_w8_s3", 14.4, 13.5),
     (LHS, (400, 53104, 16), "bm128_bn128_bk32_w4_s4_v1", 15.1, 12.9),
     (LHS, (46328, 192, 8), "bm128_bn128_bk32_w4_s4_v1", 8.1, 7.4),
+    # Skinny: one workgroup's chain over all of K.
+    (LHST, (112, 752, 2288), "bm64_bn64_bk64_w4_s4_v1", 11.3, 8.6),
+    (LHST, (120, 1248, 2128), "bm64_bn64_bk64_w4_s4_v1", 10.6, 8.8),
+    (LHST, (128, 1352, 2312), "bm64_bn64_bk64_w4_s4_v1", 10.1, 9.1),
+    (LHS, (80, 5928, 2224), "bm64_bn64_bk64_w4_s4_v2", 20.6, 17.3),
+    (LHS, (104, 5384, 2456), "bm64_bn64_bk64_w4_s4_v2", 22.2, 18.9),
 ]
 
 
