@@ -624,12 +624,17 @@ mi_tile_cfg faster_of(int kernel_id, const Timed* table, int n, const Timed& old
   // 8.1 at 46328x192x8).
   const bool short_k = K < 512 && M > 128;
   const bool lhs = kernel_id == MI_KERNEL_MATMUL_LHS_RHS_BF16, lhsT = kernel_id == MI_KERNEL_MATMUL_LHST_RHS_BF16;
-  // Skinny, a split of the rules' stays one past K = 2048, where one
-  // workgroup's chain over all of K is longer than the fits say: unsplit in
-  // its place ran 0.77-1.0 x as fast on lhsT.rhs (112x752x2288 8.6 -> 11.3
-  // us; 1.28 x faster at 63 shapes with K 1300-1900) and 0.84-1.1 x on lhs.rhs
-  // (80x5928x2224 17.3 -> 20.6; 1.35 x faster at 60).
-  const bool stays_split = M <= 128 && (lhs || lhsT) && pick.split_k > 1 && K > 2048;
+  // Skinny, a split of the rules' stays one past K = 1280 (the fused kernel's
+  // at any K): one workgroup's chain over all of K costs more than the fits
+  // say, which were timed with the weight in the caches.  From HBM, as a
+  // decode step over many layers reads it, unsplit blocks in a split's place
+  // ran, on average over 24 to 79 shapes each, 1.01 x as fast on lhsT.rhs at
+  // K 1024-1280, 0.94 at 1280-1600 and 0.86 at 1600-2048 (56x1536x1856 10.1
+  // -> 12.4 us); 1.03, 0.98 and 0.84 on lhs.rhs (56x872x1592 10.1 -> 14.2);
+  // 0.80 to 0.87 on the fused kernel (24x3112x1032 9.1 -> 11.9).  From the
+  // caches they win up to K = 2048 (1.2-1.4 x) and lose past it
+  // (112x752x2288 8.6 -> 11.3, lhs.rhs 80x5928x2224 17.3 -> 20.6).
+  const bool stays_split = M <= 128 && pick.split_k > 1 && (K > 1280 || !(lhs || lhsT));
   if (short_k && lhsT && pick.block_m == 256 && pick.block_n == 256) return pick;
   double best_t = margin * fitted_time(old, pick.split_k, M, N, K);
   mi_tile_cfg best = pick;

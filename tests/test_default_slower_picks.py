@@ -1,7 +1,7 @@
 """Default picks at shapes where a block was timed slower than another one that the rules offer: not the slower block.
 
 Each entry: the shape, the slower block, and the times (us, calls back to back in interleaved rounds over three sets of
-inputs) of that block and of the faster one.
+inputs, or over as many weights as no cache holds) of that block and of the faster one.
 """
 
 import ctypes
@@ -48,6 +48,14 @@ SLOWER = [
     (LHST, (128, 1352, 2312), "bm64_bn64_bk64_w4_s4_v1", 10.1, 9.1),
     (LHS, (80, 5928, 2224), "bm64_bn64_bk64_w4_s4_v2", 20.6, 17.3),
     (LHS, (104, 5384, 2456), "bm64_bn64_bk64_w4_s4_v2", 22.2, 18.9),
+    # The same with the weight from HBM (800 MB of weights in turn).
+    (LHST, (56, 1536, 1856), "bm64_bn64_bk64_w4_s4_v1", 12.4, 10.1),
+    (LHST, (120, 1672, 1712), "bm64_bn64_bk64_w4_s4_v1", 15.0, 12.6),
+    (LHST, (88, 376, 1608), "bm64_bn64_bk64_w4_s4_v1", 12.2, 10.4),
+    (LHS, (56, 872, 1592), "bm64_bn64_bk64_w4_s4", 14.2, 10.1),
+    (LHS, (8, 136, 1816), "bm64_bn64_bk64_w4_s4", 10.3, 8.0),
+    (FUSED, (24, 3112, 1032), "bm32_bn128_bk64_w4_s4_v5", 11.9, 9.1),
+    (NO_GAMMA, (64, 1584, 1112), "bm32_bn128_bk64_w4_s4_v5", 12.1, 9.1),
 ]
 
 
