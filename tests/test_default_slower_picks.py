@@ -56,6 +56,10 @@ SLOWER = [
     (LHS, (8, 136, 1816), "bm64_bn64_bk64_w4_s4", 10.3, 8.0),
     (FUSED, (24, 3112, 1032), "bm32_bn128_bk64_w4_s4_v5", 11.9, 9.1),
     (NO_GAMMA, (64, 1584, 1112), "bm32_bn128_bk64_w4_s4_v5", 12.1, 9.1),
+    (FUSED, (24, 744, 4312), "bm32_bn128_bk64_w4_s4_v5_k8", 11.4, 9.8),
+    (FUSED, (16, 648, 5000), "bm32_bn128_bk64_w4_s4_v5_k16", 9.7, 8.9),
+    (FUSED, (16, 9728, 232), "bm32_bn128_bk64_w4_s4_v5", 5.6, 5.3),
+    (NO_GAMMA, (24, 480, 6776), "bm32_bn128_bk64_w4_s4_v5_k16", 10.8, 9.6),
 ]
 
 
