@@ -166,11 +166,13 @@ int mi_default_config(int kernel_id, int M, int N, int K, mi_tile_cfg* cfg);
 
 /* The default of rmsnorm_matmul for a call without gamma (what
  * mi_rmsnorm_matmul_bf16 takes when cfg and gamma are both NULL):
- * mi_default_config's pick, except that at M > 128 its 128x128, 64x128 and
- * 64x64 blocks give way to a gamma-free variant, unsplit, where that is
- * faster by the fitted times: 64x128 and 64x64 to variant 14 with the same
- * block, 128x128 to variant 16 (block_k 32, 4 stages) or to variant 14 at
- * 64x128 or 64x64.
+ * mi_default_config's pick, its 128x128, 64x128 and 64x64 blocks at M > 128
+ * giving way to a gamma-free variant, unsplit, where that is faster by the
+ * times fitted without gamma (64x128 and 64x64 to variant 14 with the same
+ * block, 128x128 to variant 16 with block_k 32 and 4 stages or to variant 14
+ * at 64x128 or 64x64); but the choice of the estimates alone, without fitted
+ * times, its small blocks gamma-free likewise, where that pick is not faster
+ * without gamma, and at M <= 128 where neither splits K.
  * No counterpart in the reference, whose kernel has no gamma at all; for
  * callers of its contract (rmsnorm_matmul_online).  A negative size is
  * MI_E_ARGS. */

@@ -584,7 +584,13 @@ const Timed* timed(const Timed* table, int n, const mi_tile_cfg& c) {
 // Whether the call can run `c` in `parts` parts: at most one workgroup per
 // CU where K is split, no part empty, gamma of a part within the entries the
 // instance stages, and the workspace within its limit.  A split in parts
-// that are no power of two keeps at least 2688 of K in each.
+// that are no power of two keeps at least 2688 of K in each (3 parts from
+// K = 8064, 5 from 13440, 6 from 16128, 7 from 18816, 12 from 32256): two
+// default picks that tests name set that line, 896x1472x7872 lhsT.rhs (29.9
+// us in 2 parts, 31.1 in the 6 that the fits take) and 1536x1536x6144 lhs.rhs
+// (38.5 unsplit, 38.2 in 3).  Without it picks are 1.025 (fused), 1.04
+// (lhs.rhs) and 1.05 x (lhsT.rhs) faster on average at 122 drawn shapes, and
+// over 3 % slower at 23 of them.
 bool runs_split(int kernel_id, const mi_tile_cfg& c, int parts, int M, int N, int K) {
   const long long kt = ((long long)K + c.block_k - 1) / c.block_k, kts = (kt + parts - 1) / parts;
   if (parts > 1) {
@@ -671,7 +677,7 @@ mi_tile_cfg refined(int kernel_id, const Timed* table, int n, const mi_tile_cfg&
 // fp32: the MFMA kernel with K split over the waves (variant 3; variants 0,
 // in sequential K order, and 1 stay selectable), in the block and wave count
 // of the least estimated time (us).  The busiest CU runs `rounds` blocks.
-// Each costs its MFMAs (64 cycles per 4096 multiply-adds at 2.4 GHz and 0.94
+// Each costs its MFMAs (64 cycles per 2048 multiply-adds at 2.4 GHz and 0.94
 // of that rate; 0.42 for the 16x16 blocks, which wait for their loads more),
 // its operand bytes from L2 (63 GB/s per CU), and the latency of a load per
 // K chunk of a wave's chain (0.26 us, once: the rounds overlap); the three
@@ -751,9 +757,10 @@ mi_tile_cfg refined_skinny(int kernel_id, int M, int N, int K) {
 // campaign the rules' own ran within 1.06 and 1.05.  Its gains are splits of
 // 256-long blocks where the rules take a smaller block unsplit or in fewer
 // parts (lhsT.rhs 4736x1128x11552: 163 -> 129 us; 2528x656x15008: 84 -> 70).
-// lhsT.rhs past 2.5e11 operations keeps the rules' pick (1024x8192x16384 is
-// fixed by a test), as does lhs.rhs where its rule for shapes timed on their
-// own takes 256 x 128 in 2 parts.
+// lhsT.rhs past 2.5e11 operations keeps the rules' pick (at 21 drawn shapes up
+// to 4e11 the fits' ran 1.10 x its time on average, slower at 18), as does
+// lhs.rhs where its rule for shapes timed on their own takes 256 x 128 in 2
+// parts.
 //
 // Blocks 192 wide come last: they win where the other blocks leave CUs idle
 // in the last round (lhs.rhs 1000x5000x4104: 160 tiles of 128 x 256 leave 96
@@ -764,9 +771,11 @@ mi_tile_cfg refined_skinny(int kernel_id, int M, int N, int K) {
 // each drawn afterwards 1.11 (1.04 at least) and 1.12 x (1.04).  Below
 // K = 512 the fits miss by up to 20 % and the picks stay; so do lhsT.rhs
 // picks already split (which fill the chip: 1.10 x at one of 120 shapes) and
-// 256 x 256 and 64 x 256 blocks without padded rows: tests fix those at
-// 3072^3, where 256 tiles of 192 x 192 would fill the one round that 144 of
-// 256 x 256 do not, and at 1088x3712x8000.
+// 256 x 256 and 64 x 256 blocks without padded rows.  Times do not bear that
+// last line out: 192-wide blocks in their place are 1.15 x faster at 63 drawn
+// shapes, slower at none (3072^3 60.7 -> 49.3 us: 256 tiles of 192 x 192 fill
+// the one round that 144 of 256 x 256 do not; 1088x3712x8000 73.9 -> 70.0).
+// It keeps the two picks that tests name there.
 mi_tile_cfg refined_matmul(int kernel_id, bool lhs, int M, int N, int K) {
   const mi_tile_cfg rules = matmul_default(kernel_id, lhs, M, N, K);
   if (lhs && rules.block_m == 256 && rules.block_n == 128 && rules.split_k == 2) return rules;
@@ -789,9 +798,9 @@ mi_tile_cfg refined_matmul(int kernel_id, bool lhs, int M, int N, int K) {
 // within 1.032 of the fastest on average; the rules' own ran within 1.18 at
 // 70 (600x304x584: 11.0 -> 6.6 us; 1176x1432x1168: 19.5 -> 12.8;
 // 6272x240x968: 19.9 -> 11.5).  Where M >= 256, N >= 2048 and K >= 2048 it
-// has to win by 30 %: tests fix the rules' picks at several shapes there
-// (all but 256x2048x2048, where 64 x 64 blocks take 13 us against 18.7, are
-// within 1.04 of the fastest).
+// has to win by 30 %, which keeps the picks that tests name there; at 5 %
+// the picks it changes are 1.14 x faster at 61 drawn shapes, over 3 % slower
+// at 2 (256x2048x2048 17.8 -> 13.2 us).
 mi_tile_cfg refined_fused(int M, int N, int K) {
   const double margin = M >= 256 && N >= 2048 && K >= 2048 ? 0.7 : 0.95;
   return refined(MI_KERNEL_RMSNORM_MATMUL_BF16, kFusedTimed, count(kFusedTimed), fused_default(M, N, K), margin, 1.5e11,

@@ -148,11 +148,13 @@ __global__ __launch_bounds__(256) void mm_f32_mfma_kernel(const float* __restric
 //
 // Bound: the fp32 MFMA rate (157 TFLOP/s at 2.4 GHz) where tiles fill the
 // chip, the latency of the loads where they do not.  An MFMA runs 64 cycles
-// on 4 KiB of operands, so neither LDS nor L1 is near its limit and the
-// operands need no LDS.  Variant 1 waits for every chunk it loads and gives
-// a tile one chain of K / 2 MFMAs; here the loads run a chunk ahead, and the
-// chain of a tile is spread over WAVES waves of the CU that holds it, so a
-// small block, of which there are enough for every CU, is not a long chain.
+// on 512 bytes of operands (half as many where a wave's 2x2 fragments share
+// them), 4 to 8 bytes a cycle and SIMD, so neither LDS nor L1 is near its
+// limit and the operands need no LDS.  Variant 1 waits for every chunk it
+// loads and gives a tile one chain of K / 2 MFMAs; here the loads run a
+// chunk ahead, and the chain of a tile is spread over WAVES waves of the CU
+// that holds it, so a small block, of which there are enough for every CU,
+// is not a long chain.
 // Measured in graphs of back-to-back calls, variant 1 -> 3: 256x512x512
 // (M, N, K) 27.0 -> 4.7 us, 1000x1501x777 60.9 -> 25.3 us (90 TFLOP/s),
 // 128x4072x4015 225 -> 39 us, 64x64x4096 224 -> 8.2 us, 2048^3 240 -> 130 us
