@@ -697,7 +697,11 @@ mi_tile_cfg f32_default(int M, int N, int K) {
   mi_tile_cfg best = cands[0];
   double best_t = 0.0;
   for (const mi_tile_cfg& c : cands) {
-    const double rounds = (double)((tiles_of(M, N, c.block_m, c.block_n) + kCUs - 1) / kCUs);
+    const long long tiles = tiles_of(M, N, c.block_m, c.block_n);
+    // A launch holds fewer than 2^32 threads; 64x64 blocks of 4 waves, as
+    // many outputs a thread as variant 1's, take what variant 1 took.
+    if (&c != cands && tiles * c.waves * 64 >= (1LL << 32)) continue;
+    const double rounds = (double)((tiles + kCUs - 1) / kCUs);
     const double chain = (double)(((K + c.block_k - 1) / c.block_k + c.waves - 1) / c.waves);  // chunks per wave
     const double area = (double)c.block_m * c.block_n;
     const double mfma = rounds * chain * (c.waves / 4) * c.block_k * area / 32.0 / 2400.0 / (c.block_m == 16 ? 0.42 : 0.94);
