@@ -222,6 +222,23 @@ PyObject* remember(PyObject*, PyObject* args) {
   Py_RETURN_NONE;
 }
 
+// knows(kind, M, N, K): whether remember() has this shape's config for the
+// library in use.  The Python body asks after each call it runs, so that the
+// calls it always runs (a mode, a subclass, a view) bind and remember once.
+PyObject* knows(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  if (n != 4) {
+    PyErr_SetString(PyExc_TypeError, "knows takes 4 arguments");
+    return nullptr;
+  }
+  long long v[4];
+  for (int i = 0; i < 4; ++i) {
+    v[i] = PyLong_AsLongLong(args[i]);
+    if (v[i] == -1 && PyErr_Occurred()) return nullptr;
+  }
+  const char* env = std::getenv("MI_KERNELS_LIB");
+  return PyBool_FromLong(g_lib.check_rc && g_lib.env == (env ? env : "") && g_configs.count(Shape{v[0], v[1], v[2], v[3]}));
+}
+
 // forget(): drop every shape's config (the tuned table changed).
 PyObject* forget(PyObject*, PyObject*) {
   g_configs.clear();
@@ -231,6 +248,7 @@ PyObject* forget(PyObject*, PyObject*) {
 PyMethodDef kMethods[] = {{"call", (PyCFunction)(void (*)(void))call, METH_FASTCALL, nullptr},
                           {"bind", bind, METH_VARARGS, nullptr},
                           {"remember", remember, METH_VARARGS, nullptr},
+                          {"knows", (PyCFunction)(void (*)(void))knows, METH_FASTCALL, nullptr},
                           {"forget", forget, METH_NOARGS, nullptr},
                           {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_torch_call", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};

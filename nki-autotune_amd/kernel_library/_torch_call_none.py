@@ -20,5 +20,9 @@ def remember(*shape_and_config):
     return None
 
 
+def knows(kind, M, N, K):
+    return True  # nothing to remember
+
+
 def forget():
     return None

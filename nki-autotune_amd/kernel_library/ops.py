@@ -42,7 +42,10 @@ _LHST, _LHST_F32, _RMS, _LHS, _RMS_NO_GAMMA = range(5)
 
 
 def _remember(kind: int, M: int, N: int, K: int, cfg: TileConfig) -> None:
-    """Hand the native call the config that this shape has just run with, and the library that ran it."""
+    """Hand the native call the config that this shape has just run with, and the library that ran it (once: a call
+    that the native one leaves to Python each time pays 0.2 us here, and 7.6 for a new shape)."""
+    if _torch_call.knows(kind, M, N, K):
+        return
     L = _lib.lib()
     fns = (L.mi_matmul_lhsT_rhs_bf16, L.mi_matmul_lhsT_rhs_f32, L.mi_rmsnorm_matmul_bf16, L.mi_matmul_lhs_rhs_bf16)
     _torch_call.bind(os.environ.get("MI_KERNELS_LIB", ""), *(ctypes.cast(f, ctypes.c_void_p).value for f in fns),
