@@ -12,8 +12,10 @@
 #include <string.h>
 
 #include <atomic>
+#include <chrono>
 #include <map>
 #include <mutex>
+#include <thread>
 #include <unordered_map>
 #include <utility>
 #include <vector>
@@ -295,6 +297,7 @@ int zero_output(void* out, size_t n, void* stream) {
 constexpr uint64_t kPoolKeepBytes = 256ull << 20;
 std::mutex g_pool_mu;
 std::map<int, hipMemPool_t> g_pools;
+std::atomic<bool> g_freed{false};  // a workspace was freed since mi_release_workspace last waited for the frees
 
 int workspace_pool(hipMemPool_t* out) {
   int dev = 0;
@@ -348,6 +351,7 @@ int run_pooled(const mi::MiEntry* e, const mi_tile_cfg& cfg, const mi::MiArgs& a
   if (ae != hipSuccess) return hip_fail(ae, "workspace alloc");
   const int lrc = launch(e, cfg, a, ws, false, stream);
   const hipError_t fe = hipFreeAsync(ws, (hipStream_t)stream);
+  g_freed = true;
   if (lrc != MI_OK) return lrc;
   if (fe != hipSuccess) return hip_fail(fe, "workspace free");
   return MI_OK;
@@ -412,6 +416,7 @@ int run_kept(const mi::MiEntry* e, const mi_tile_cfg& cfg, const mi::MiArgs& a, 
   }
   if (k->bytes < ws_bytes) {
     if (k->ptr && (err = hipFreeAsync(k->ptr, stream)) != hipSuccess) return hip_fail(err, "workspace free");
+    if (k->ptr) g_freed = true;
     k->ptr = nullptr;
     k->bytes = 0;
     // Round up (to 1 MiB, at least 1/4 more) so that growing shapes reallocate rarely.
@@ -640,6 +645,7 @@ int mi_release_workspace(void) {
       rc = hip_fail(e, "releasing a kept workspace");
       break;
     }
+    if (k.ptr) g_freed = true;
     k.ptr = nullptr;
   }
   if (rc != MI_OK) {
@@ -660,6 +666,20 @@ int mi_release_workspace(void) {
         (e = hipMemPoolTrimTo(kv.second, 0)) != hipSuccess) {
       rc = hip_fail(e, "releasing the workspace pool");
       break;
+    }
+  }
+  // A device's free memory follows its frees about 1 ms later, so a caller
+  // that looks at it at once read the old figure after half of 400 releases
+  // of 1 GiB: where something was freed, wait until it stands still for 3 ms
+  // (30 ms at most, as others may allocate meanwhile).
+  if (rc == MI_OK && g_freed.exchange(false)) {
+    for (const auto& kv : g_pools) {
+      size_t last = 0, now = 0, total = 0;
+      if (hipSetDevice(kv.first) != hipSuccess) continue;
+      for (int i = 0; i < 10 && hipMemGetInfo(&now, &total) == hipSuccess && (i == 0 || now != last); ++i) {
+        last = now;
+        std::this_thread::sleep_for(std::chrono::milliseconds(3));
+      }
     }
   }
   e = hipSetDevice(cur);
